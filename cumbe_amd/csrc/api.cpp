@@ -6,6 +6,7 @@
 #include <iterator>
 #include <chrono>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -233,7 +234,8 @@ mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_hos
     kp.sparse_ratio = tu.sparse_ratio;
     kp.split_nodes = tu.split_nodes;
     kp.twins = (tu.flags & MBE_FLAG_REFERENCE_TREE) ? 0 : 1;
-    HIPC(hipHostGetDevicePointer((void**)&kp.abort, abort_host, 0));
+    if (tu.max_nodes || tu.time_limit_ms > 0)
+        HIPC(hipHostGetDevicePointer((void**)&kp.abort, abort_host, 0));
     kp.node_count = kp.stats + mbe::kStatNodeBudget;
     kp.node_budget = tu.max_nodes;
     kp.overflow_list = ovf_list;
@@ -244,7 +246,7 @@ mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_hos
     kp.slot_words = slot_words;
     kp.n_slots = kSlots;
     kp.dq = B.dq.as<unsigned long long>();
-    HIPC(hipHostGetDevicePointer((void**)&kp.progress, B.progress, 0));
+    if (getenv("MBE_PROGRESS")) HIPC(hipHostGetDevicePointer((void**)&kp.progress, B.progress, 0));
     return MBE_OK;
 }
 
@@ -839,7 +841,8 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
         kp.sparse_ratio = tu.sparse_ratio;
         kp.split_nodes = tu.split_nodes;
         kp.twins = (tu.flags & MBE_FLAG_REFERENCE_TREE) ? 0 : 1;
-        HIPC(hipHostGetDevicePointer((void**)&kp.abort, E.abort_flag, 0));
+        if (tu.max_nodes || tu.time_limit_ms > 0)
+            HIPC(hipHostGetDevicePointer((void**)&kp.abort, E.abort_flag, 0));
         kp.node_count = kp.stats + mbe::kStatNodeBudget;
         kp.node_budget = tu.max_nodes;
         kp.overflow_list = lists + (pass & 1) * w_list;

@@ -32,6 +32,8 @@ enum KStat : int {
     kStatDropped = 6,    // slots discarded (snapshot did not fit the thief's arena)
     kStatNodeBudget = 7, // nodes charged against the watchdog budget
     kStatWords = 8,      // bit-matrix operand words the nodes read (algorithmic)
+    kStatAbortSeen = 9,  // watchdog: device mirror of the abort flag
+    kStatAbortPoll = 10, // and the clock of its next refresh
     kStatCount = 12
 };
 
@@ -130,10 +132,12 @@ struct KParams {
     uint32_t donate_interval;   // nodes between a worker's donation checks
     uint32_t split_nodes;       // a task past this many nodes donates while the deque is short (0 = never)
     unsigned long long* dq;     // [0] head, [1] tail, [2] idle, [3] pending, [4..] seq per slot
-    // host-mapped progress: 2 slots per worker (roots done, nodes), plain stores
+    // host-mapped progress: 2 slots per worker (roots done, nodes), plain
+    // stores; null unless the host reports it
     unsigned long long* progress;
     unsigned long long* sections;   // kSecCount tick sums, or null
-    // watchdog: abort flag (host-mapped, system scope) and node budget
+    // watchdog: abort flag (host-mapped, system scope; null without one) and
+    // node budget
     unsigned long long* abort;
     unsigned long long* node_count;
     uint64_t node_budget;           // 0 = unlimited

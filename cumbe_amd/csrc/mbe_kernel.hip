@@ -129,22 +129,49 @@ __device__ __forceinline__ u64 red_add64(u64 v) {
 
 __device__ __forceinline__ void wsync() { __syncthreads(); }
 
-// Watchdog: the host (time limit) or any worker (node budget) raises
-// *abort; workers then drop their work and drain the deque. Checked every
-// kAbortEvery nodes.
-constexpr uint32_t kAbortEvery = 256;
+__device__ __forceinline__ u64 ld_rlx(unsigned long long* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_rel(unsigned long long* p, u64 v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_rlx(unsigned long long* p, u64 v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Watchdog: the host (time limit) or any worker (node budget) raises an
+// abort flag; workers then drop their work and drain the deque. Without a
+// watchdog kp.abort is null. The host's flag lies in host memory, a link
+// round trip away: the workers look at a mirror in device memory, which one
+// of them refreshes every kAbortPollTicks.
+constexpr uint32_t kAbortEvery = 256;      // nodes between a worker's checks
+constexpr uint64_t kAbortPollTicks = 2000; // 20 us of the 100 MHz clock
 __device__ __forceinline__ bool aborted(const KParams& kp) {
+    if (kp.serve) return uni64(lane() == 0 ? ld_rlx(&kp.serve->abort_seen) : 0) != 0;
     if (!kp.abort) return false;
     u64 a = 0;
-    if (lane() == 0) a = __hip_atomic_load(kp.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (lane() == 0) {
+        unsigned long long* seen = kp.stats + kStatAbortSeen;
+        unsigned long long* next = kp.stats + kStatAbortPoll;
+        a = ld_rlx(seen);
+        if (!a) {
+            const u64 t = ld_rlx(next), now = (u64)wall_clock64();
+            if (now >= t && atomicCAS(next, t, now + kAbortPollTicks) == t) {
+                a = __hip_atomic_load(kp.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                if (a) st_rlx(seen, 1ull);
+            }
+        }
+    }
     return uni64(a) != 0;
 }
 __device__ __forceinline__ bool charge_nodes(const KParams& kp, u64 n) {
     u64 total = 0;
     if (lane() == 0 && kp.node_budget) {
         total = atomicAdd(kp.node_count, n) + n;
-        if (total >= kp.node_budget)
+        if (total >= kp.node_budget) {
+            st_rlx(kp.stats + kStatAbortSeen, 1ull);
             __hip_atomic_store(kp.abort, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
     return aborted(kp);
 }
@@ -944,15 +971,6 @@ __device__ __noinline__ u64 prune_twins(u64* F, const u64* Lc, const u64* cols, 
 // then hl[d], hc[nc], rows[nc * W], P[Wc], Q[Wc]: a LEVEL(L, R, P, Q) call
 // over a compacted universe (L = all d bits).
 
-__device__ __forceinline__ u64 ld_rlx(unsigned long long* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_rel(unsigned long long* p, u64 v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_rlx(unsigned long long* p, u64 v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // Acquire-only fence: waits for this wave's memory operations and
 // invalidates its stale cache lines, without writing the L2 back (a release
 // or a full fence would write back every dirty line of the XCD's L2).
@@ -2241,9 +2259,7 @@ __global__ __launch_bounds__(64) void mbe_persistent(KParams kp) {
     sec.init(kp.sections != nullptr, lds_mem);
     for (;;) {
         wsync();
-        // served kernels poll the device mirror of the host's abort flag
-        const bool stop =
-            kp.serve ? uni64(lane() == 0 ? ld_rlx(&kp.serve->abort_seen) : 0) != 0 : aborted(kp);
+        const bool stop = aborted(kp);
         if (stop) roots_left = false;
         if (roots_left) {
             u64 t = 0;

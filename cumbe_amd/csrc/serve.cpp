@@ -155,6 +155,7 @@ struct mbe_server {
         kp.serve = sctl.as<mbe::ServeCtl>();
         kp.mail_cap = cfg.table_cap;
         kp.data = data.as<uint64_t>();
+        HIPC(hipHostGetDevicePointer((void**)&kp.abort, abort_flag, 0));
         HIPC(hipHostGetDevicePointer((void**)&kp.done, done, 0));
         HIPC(hipHostGetDevicePointer((void**)&kp.mail, mail, 0));
         HIPC(hipHostGetDevicePointer((void**)&kp.mail_pub, mail_pub, 0));
