@@ -185,19 +185,27 @@ hipError_t wait_with_progress(Engine& E, const Bufs& B, uint32_t nw, uint64_t n_
 // Size the buffers of one pass and fill its kernel parameters. The task list
 // (explicit global task ids, or none for all tasks) is copied to the device.
 mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_host, const Meta& m,
-                      const Tune& tu, int variant, const std::vector<uint64_t>& task_list,
-                      uint64_t n_tasks, uint64_t arena_words, uint32_t workers, mbe::KParams& kp) {
+                      const Tune& tu, int variant, bool first,
+                      const std::vector<uint64_t>& task_list, uint64_t n_tasks,
+                      uint64_t arena_words, uint32_t workers, mbe::KParams& kp) {
     HIPC(B.ctl.ensure(m.ctl_words() * 8));
     const uint64_t ovf_cap = std::max<uint64_t>(m.total_tasks, 1);
     HIPC(B.ovf.ensure(ovf_cap * 8 * 2));
     HIPC(B.arena.ensure(arena_words * workers * 8));
     HIPC(B.mark.ensure(m.mark_words() * workers * 8));
     HIPC(B.cpos.ensure(m.cpos_len() * workers * 4));
-    // a slot holds a compacted level of any problem that fits an arena, up
-    // to 4 MiB per slot
+    // the general engine's ring: a slot holds a compacted level of any problem
+    // that fits an arena, up to 4 MiB per slot; the tree engine's hand-over: a
+    // slot per worker
+    const bool tree = first && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
     const uint64_t slot_words = std::min<uint64_t>(std::max<uint64_t>(4096, arena_words), 1u << 19);
-    HIPC(B.slots.ensure((size_t)kSlots * slot_words * 8));
-    HIPC(B.dq.ensure((4 + (size_t)kSlots) * 8));
+    if (tree) {
+        HIPC(B.tctl.ensure((size_t)mbe::tree_ctl_words(workers) * 8));
+        HIPC(B.tslots.ensure(tree_slot_words(arena_words) * workers * 8));
+    } else {
+        HIPC(B.slots.ensure((size_t)kSlots * slot_words * 8));
+        HIPC(B.dq.ensure((4 + (size_t)kSlots) * 8));
+    }
     HIPC(B.ensure_progress(workers));
     memset(B.progress, 0, 2 * (size_t)workers * 8);
     unsigned long long* ctl = B.ctl.as<unsigned long long>();
@@ -234,6 +242,11 @@ mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_hos
     kp.sparse_ratio = tu.sparse_ratio;
     kp.split_nodes = tu.split_nodes;
     kp.twins = (tu.flags & MBE_FLAG_REFERENCE_TREE) ? 0 : 1;
+    kp.tree = tree;
+    kp.tctl = B.tctl.as<unsigned long long>();
+    kp.tslots = B.tslots.as<uint64_t>();
+    kp.tslot_words = tree_slot_words(arena_words);
+    kp.tworkers = workers;
     if (tu.max_nodes || tu.time_limit_ms > 0)
         HIPC(hipHostGetDevicePointer((void**)&kp.abort, abort_host, 0));
     kp.node_count = kp.stats + mbe::kStatNodeBudget;
@@ -257,9 +270,13 @@ mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_hos
 hipError_t enqueue_pass(const mbe::KParams& kp, uint32_t workers, size_t ctl_clear,
                         hipStream_t s) {
     hipError_t e = mbe::launch_fill(kp.cursor, ctl_clear, 0ull, s);
-    if (e == hipSuccess)
-        e = mbe::launch_fill((unsigned long long*)kp.mark, kp.mark_words * workers, 0ull, s);
-    if (e == hipSuccess) e = mbe::launch_dq_init(kp.dq, kp.n_slots, s);
+    if (kp.tree) {
+        if (e == hipSuccess) e = mbe::launch_fill(kp.tctl, mbe::tree_ctl_words(workers), 0ull, s);
+    } else {
+        if (e == hipSuccess)
+            e = mbe::launch_fill((unsigned long long*)kp.mark, kp.mark_words * workers, 0ull, s);
+        if (e == hipSuccess) e = mbe::launch_dq_init(kp.dq, kp.n_slots, s);
+    }
     if (e == hipSuccess) e = mbe::launch_mbe(kp, workers, s);
     return e;
 }
@@ -312,8 +329,8 @@ mbe_status run_tasks(Engine& E, Bufs& B, const Meta& m, int variant, const Tune&
             HIPC(hipEventRecord(E.ev0, E.stream));
             HIPC(hipGraphLaunch(pre->exec, E.stream));
         } else {
-            mbe_status s = setup_pass(B, E.stream, E.abort_flag, m, tu, variant, task_list, n_tasks,
-                                      arena_words, nw, kp);
+            mbe_status s = setup_pass(B, E.stream, E.abort_flag, m, tu, variant, pass == 0,
+                                      task_list, n_tasks, arena_words, nw, kp);
             if (s != MBE_OK) return s;
             if (em) {
                 kp.emit_pos = em->pos;
@@ -800,9 +817,14 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
         if (pass > 6) return fail(MBE_ERANGE, "root subproblem does not fit an arena of the scratch");
         const uint64_t slot_words = std::min<uint64_t>(std::max<uint64_t>(4096, arena_words), 1u << 19);
         const uint64_t w_slots = up4(kNoAllocSlots * slot_words);
-        const uint64_t per_worker = up4(arena_words) + up4(m.mark_words()) + up4((m.cpos_len() + 1) / 2);
-        const uint64_t fit = fixed + w_slots < mbe::kNoAllocWords
-                                 ? (mbe::kNoAllocWords - fixed - w_slots) / per_worker : 0;
+        const bool tree = pass == 0 && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
+        // the tree engine's hand-over: a slot and, of the control block, a
+        // flag line and a share of the idle map per worker
+        const uint64_t tslot_words = std::min(tree_slot_words(arena_words), kNoAllocTreeSlotWords);
+        const uint64_t per_worker = up4(arena_words) + up4(m.mark_words()) +
+                                    up4((m.cpos_len() + 1) / 2) + (tree ? tslot_words + 32 : 0);
+        const uint64_t fit = fixed + w_slots + 64 < mbe::kNoAllocWords
+                                 ? (mbe::kNoAllocWords - fixed - w_slots - 64) / per_worker : 0;
         if (fixed_workers && pass == 0 && workers > fit)
             return fail(MBE_ERANGE, std::to_string(workers) + " workers need " +
                                         std::to_string((fixed + w_slots + workers * per_worker) * 8) +
@@ -816,6 +838,7 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
         uint64_t* arena = slots + w_slots;
         uint64_t* mark = arena + (uint64_t)nw * up4(arena_words);
         uint32_t* cpos = (uint32_t*)(mark + (uint64_t)nw * up4(m.mark_words()));
+        uint64_t* tslots = (uint64_t*)cpos + (uint64_t)nw * up4((m.cpos_len() + 1) / 2);
         kp = mbe::KParams{};
         kp.graphs = gdev;
         kp.n_graphs = 1;
@@ -841,6 +864,11 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
         kp.sparse_ratio = tu.sparse_ratio;
         kp.split_nodes = tu.split_nodes;
         kp.twins = (tu.flags & MBE_FLAG_REFERENCE_TREE) ? 0 : 1;
+        kp.tree = tree;
+        kp.tslots = tslots;
+        kp.tslot_words = tslot_words;
+        kp.tctl = (unsigned long long*)(tslots + (uint64_t)nw * tslot_words);
+        kp.tworkers = nw;
         if (tu.max_nodes || tu.time_limit_ms > 0)
             HIPC(hipHostGetDevicePointer((void**)&kp.abort, E.abort_flag, 0));
         kp.node_count = kp.stats + mbe::kStatNodeBudget;
@@ -929,8 +957,8 @@ mbe_status capture_pass0(Engine& E, mbe_batch_plan* p) {
         for (uint64_t r = p->tu.root_begin; r < end; r += p->tu.root_stride) task_list.push_back(r);
         n_tasks = task_list.size();
     }
-    mbe_status s = setup_pass(p->b, E.stream, E.abort_flag, p->m, p->tu, p->variant, task_list,
-                              n_tasks, p->tu.arena_words, p->tu.workers, p->pass0.kp);
+    mbe_status s = setup_pass(p->b, E.stream, E.abort_flag, p->m, p->tu, p->variant, true,
+                              task_list, n_tasks, p->tu.arena_words, p->tu.workers, p->pass0.kp);
     if (s != MBE_OK) return s;
     p->pass0.workers = p->tu.workers;
     HIPC(hipStreamSynchronize(E.stream));
@@ -950,8 +978,11 @@ bool capture_current(const mbe_batch_plan* p) {
     return p->pass0.exec && kp.arena == p->b.arena.as<uint64_t>() &&
            kp.mark == p->b.mark.as<uint64_t>() && kp.cpos == p->b.cpos.as<uint32_t>() &&
            kp.cursor == p->b.ctl.as<unsigned long long>() &&
-           kp.overflow_list == p->b.ovf.as<uint64_t>() && kp.slots == p->b.slots.as<uint64_t>() &&
-           kp.dq == p->b.dq.as<unsigned long long>();
+           kp.overflow_list == p->b.ovf.as<uint64_t>() &&
+           kp.slots == p->b.slots.as<uint64_t>() &&
+           kp.dq == p->b.dq.as<unsigned long long>() &&
+           kp.tctl == p->b.tctl.as<unsigned long long>() &&
+           kp.tslots == p->b.tslots.as<uint64_t>();
 }
 
 }  // namespace

@@ -67,6 +67,26 @@ constexpr uint64_t kNoAllocWords = kNoAllocBytes / 8;
 // u64 words; a worker's LDS budget is at least this plus one frame.
 constexpr uint32_t kLdsHeaderWords = 344;
 
+// Control block of the tree engine's hand-over (see mbe_tree.h): a line of 16
+// u64 words each for the active count, 64 workers' idle bits and a worker's
+// flag.
+constexpr uint32_t tree_ctl_words(uint32_t workers) {
+    return 16 * (1 + (workers + 63) / 64 + workers);
+}
+
+// Arena words that a wide level of the tree engine can take: W words of L, nc
+// candidates, np of them in P or X (tile stack, hash terms, reduction scratch,
+// rows, frames; nothing in LDS).
+constexpr uint64_t tree_wide_words(uint64_t W, uint64_t nc, uint64_t np) {
+    const uint64_t wc = (nc + 63) / 64;
+    return 66 * 13 + 64 * W * 3 + nc + wc * 64 * W + (nc + 1) / 2 + (np + 2) * (4 + W + 3 * wc);
+}
+// and a root of degree d with nc candidates: its candidate lists and rows too
+constexpr uint64_t tree_root_words(uint64_t d, uint64_t nc) {
+    const uint64_t W = (d + 63) / 64;
+    return (nc + 1) / 2 + nc + 1 + tree_wide_words(W, nc, nc < d ? nc : d) + nc * W;
+}
+
 // Deque slot header for donated subtrees (see mbe_kernel.hip).
 constexpr uint32_t kSlotHeaderWords = 8;
 
@@ -119,7 +139,8 @@ struct KParams {
     uint32_t list_cutoff;       // |P|+|Q| at or below which a node tests rows (forward form)
     uint32_t sparse_ratio;      // list-mode roots: bitmap words > ratio * local adjacency (0 = never)
     uint32_t compact_ratio;     // re-localise a child whose universe shrank this much (0 = never)
-    uint32_t twins;             // nonzero: drop twin candidates of the selected vertex from P
+    uint32_t twins;             // nonzero: drop candidates that cannot give a maximal biclique
+    uint32_t tree;              // nonzero: the tree engine runs this pass (needs twins)
     // roots that did not fit the arena
     unsigned long long* overflow_count;
     uint64_t* overflow_list;
@@ -132,6 +153,12 @@ struct KParams {
     uint32_t donate_interval;   // nodes between a worker's donation checks
     uint32_t split_nodes;       // a task past this many nodes donates while the deque is short (0 = never)
     unsigned long long* dq;     // [0] head, [1] tail, [2] idle, [3] pending, [4..] seq per slot
+    // the tree engine's hand-over: control block (tree_ctl_words) and one slot
+    // per worker
+    unsigned long long* tctl;
+    uint64_t* tslots;               // tworkers * tslot_words
+    uint64_t tslot_words;
+    uint32_t tworkers;
     // host-mapped progress: 2 slots per worker (roots done, nodes), plain
     // stores; null unless the host reports it
     unsigned long long* progress;

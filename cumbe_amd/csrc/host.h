@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -60,7 +61,7 @@ struct DevBuf {
 // Device buffers of one launch context: the engine's (reused by every solve)
 // or a batch plan's (owned by the plan, whose captured graph points into them).
 struct Bufs {
-    DevBuf arena, mark, cpos, ctl, graphs, data, ovf, slots, dq, busy;
+    DevBuf arena, mark, cpos, ctl, graphs, data, ovf, slots, dq, busy, tctl, tslots;
     unsigned long long* progress = nullptr;  // host-mapped, 2 per worker
     size_t progress_slots = 0;
     hipError_t ensure_progress(size_t workers) {
@@ -74,7 +75,8 @@ struct Bufs {
         return e;
     }
     void release() {
-        for (DevBuf* b : {&arena, &mark, &cpos, &ctl, &graphs, &data, &ovf, &slots, &dq, &busy}) {
+        for (DevBuf* b : {&arena, &mark, &cpos, &ctl, &graphs, &data, &ovf, &slots, &dq, &busy, &tctl,
+                          &tslots}) {
             if (b->p) (void)hipFree(b->p);
             b->p = nullptr;
             b->bytes = 0;
@@ -102,13 +104,21 @@ struct Meta {
     uint32_t ng = 0;
     uint32_t max_nr = 1;
     uint64_t total_tasks = 0;
-    uint64_t mark_words() const { return (max_nr + 63) / 64 + 1; }
+    // whole blocks of four words (see marked_below)
+    uint64_t mark_words() const { return ((uint64_t)max_nr + 255) / 256 * 4; }
     uint64_t cpos_len() const { return (uint64_t)max_nr + 1; }
     // control block: cursor, overflow count, stats, section ticks, results
     size_t ctl_words() const { return 2 + mbe::kStatCount + mbe::kSecCount + 2 * (size_t)ng; }
 };
 
 constexpr uint32_t kSlots = 1024;  // deque slots
+// words of a worker's hand-over slot (tree engine), at most: a level of 2,000
+// candidates over 1,024 L bits; larger levels are not handed over
+constexpr uint64_t kTreeSlotWords = 1u << 16;
+inline uint64_t tree_slot_words(uint64_t arena_words) {
+    return std::min<uint64_t>(std::max<uint64_t>(1024, arena_words), kTreeSlotWords);
+}
+constexpr uint64_t kNoAllocTreeSlotWords = 4096;
 // allocation-free solve: deque slots and default arena (u64 words)
 constexpr uint32_t kNoAllocSlots = 64;
 constexpr uint64_t kNoAllocArenaWords = 1u << 15;
@@ -129,10 +139,13 @@ mbe_status upload(Bufs& B, hipStream_t stream, const std::vector<const Prepared*
 Meta meta_of(const std::vector<const Prepared*>& ps, uint64_t total_tasks);
 
 // Size the buffers of one pass and fill its kernel parameters; abort_host is
-// the host-mapped watchdog flag the kernel polls.
+// the host-mapped watchdog flag the kernel polls. first: the first pass, which
+// the tree engine runs unless the reference's tree is asked for; later passes
+// run what it left on the general engine.
 mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_host, const Meta& m,
-                      const Tune& tu, int variant, const std::vector<uint64_t>& task_list,
-                      uint64_t n_tasks, uint64_t arena_words, uint32_t workers, KParams& kp);
+                      const Tune& tu, int variant, bool first,
+                      const std::vector<uint64_t>& task_list, uint64_t n_tasks,
+                      uint64_t arena_words, uint32_t workers, KParams& kp);
 
 // Enqueue one pass with kernels only (capturable): clear control words and
 // marks, reset the deque, launch the persistent workers.

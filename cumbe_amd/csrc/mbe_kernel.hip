@@ -1558,9 +1558,9 @@ __device__ bool try_donate(const KParams& kp, const Local& S, uint32_t cur, uint
 // SP: the outermost problem may be a list-mode root (its children are bit
 // matrices); without it the node loop holds no list-mode code.
 template <int V, bool SP>
-__device__ void dfs(const KParams& kp, const DevGraph& G, uint32_t g, Local& S, u64* arena,
-                    u64* lds, uint32_t* premin, u64& cnt, u64& hs, u64& nodes, u64& donated,
-                    u64& words, Sec& sec) {
+__device__ __noinline__ void dfs(const KParams& kp, const DevGraph& G, uint32_t g, Local& S,
+                                 u64* arena, u64* lds, uint32_t* premin, u64& cnt, u64& hs,
+                                 u64& nodes, u64& pruned, u64& donated, u64& words, Sec& sec) {
     u64* nest = lds + kLdsNest;
     uint32_t np = 0, depth0 = 0, k = 1;
     const u64 split_at = kp.split_nodes ? nodes + kp.split_nodes : ~0ull;
@@ -1639,6 +1639,7 @@ __device__ void dfs(const KParams& kp, const DevGraph& G, uint32_t g, Local& S, 
             words += (o.has_tw ? 0 : (u64)S.Wc * (nl + 1)) + (r >> 32) * S.W;
         }
         sec.mark(o.maximal ? kSecExpand : kSecCheck);
+        if (!o.maximal) pruned++;
         if (o.maximal) {
             const u64 sl = sum_l(S, nl);
             const u64 sr = F[1] + S.hc[xk] + o.abh;
@@ -1801,8 +1802,9 @@ __device__ __noinline__ int build_root_sparse(const KParams& kp, const DevGraph&
 template <int V>
 __device__ __noinline__ void dfs_sparse(const KParams& kp, const DevGraph& G, uint32_t g, Local& S,
                                         u64* arena, u64* lds, uint32_t* premin, u64& cnt, u64& hs,
-                                        u64& nodes, u64& donated, u64& words, Sec& sec) {
-    dfs<V, true>(kp, G, g, S, arena, lds, premin, cnt, hs, nodes, donated, words, sec);
+                                        u64& nodes, u64& pruned, u64& donated, u64& words,
+                                        Sec& sec) {
+    dfs<V, true>(kp, G, g, S, arena, lds, premin, cnt, hs, nodes, pruned, donated, words, sec);
 }
 
 // Localise root x (rows/cols over N(x) x distance-two candidates) and
@@ -2092,7 +2094,7 @@ __device__ bool serve_claim(const KParams& kp, uint32_t wid, uint32_t& g, uint32
 // the device data buffer, appends its descriptor to the graph table and its
 // roots to the task space, then publishes the new counts (release) and
 // reports the records taken to the host. Returns true if it loaded any.
-__device__ bool serve_load(const KParams& kp) {
+__device__ __forceinline__ bool serve_load(const KParams& kp) {
     ServeCtl* sc = kp.serve;
     u64 pub = 0, taken = 0;
     if (lane() == 0) {
@@ -2193,7 +2195,7 @@ __device__ bool serve_load(const KParams& kp) {
 // An idle serving wave leaves when nothing is pending and either the
 // watchdog fired or the host closed the mailbox and every published record
 // has been loaded and every task claimed.
-__device__ bool serve_exit(const KParams& kp, u64 pend, bool stop) {
+__device__ __forceinline__ bool serve_exit(const KParams& kp, u64 pend, bool stop) {
     if (pend != 0) return false;
     u64 ex = 0;
     if (lane() == 0) {
@@ -2220,7 +2222,7 @@ __device__ bool serve_exit(const KParams& kp, u64 pend, bool stop) {
 // Donations add open tasks before they are published (try_donate), and the
 // donor's own task stays open meanwhile, so the count cannot reach zero
 // early. Roots deferred for a larger arena stay open until their pass.
-__device__ void finish_task(const KParams& kp, uint32_t g, bool failed) {
+__device__ __forceinline__ void finish_task(const KParams& kp, uint32_t g, bool failed) {
     if (!kp.remaining || lane() != 0) return;
     unsigned long long* rem = kp.remaining + 2 * (size_t)g;
     if (failed) atomicOr(rem + 1, 1ull);
@@ -2252,6 +2254,7 @@ __global__ __launch_bounds__(64) void mbe_persistent(KParams kp) {
     uint32_t* premin = (uint32_t*)(lds_mem + kLdsPreMin);
     for (uint32_t i = lane(); i < kPreMinLevels; i += 64) premin[i] = 1;  // src/main.cu:86
     u64 nodes = 0, roots = 0, build = 0, ovf = 0, donated = 0, stolen = 0, dropped = 0, words = 0;
+    u64 pruned = 0;  // non-maximal vertices taken: no nodes of the pruned tree
     bool roots_left = true, idle = false;
     uint32_t backoff = 1;
     unsigned long long* pending = kp.dq + 3;
@@ -2298,11 +2301,11 @@ __global__ __launch_bounds__(64) void mbe_persistent(KParams kp) {
                                              nodes, build);
                 sec.mark(kSecBuild);
                 if (st > 0 && S.sparse)
-                    dfs_sparse<V>(kp, G, g, S, arena, lds_mem, premin, cnt, hs, nodes, donated, words,
-                                  sec);
+                    dfs_sparse<V>(kp, G, g, S, arena, lds_mem, premin, cnt, hs, nodes, pruned, donated,
+                                  words, sec);
                 else if (st > 0)
-                    dfs<V, false>(kp, G, g, S, arena, lds_mem, premin, cnt, hs, nodes, donated, words,
-                                  sec);
+                    dfs<V, false>(kp, G, g, S, arena, lds_mem, premin, cnt, hs, nodes, pruned, donated,
+                                  words, sec);
                 if (st < 0) {
                     ovf++;
                     if (lane() == 0) {
@@ -2357,8 +2360,8 @@ __global__ __launch_bounds__(64) void mbe_persistent(KParams kp) {
                     const DevGraph G = kp.graphs[g];
                     u64 cnt = 0, hs = 0;
                     stolen++;
-                    dfs<V, false>(kp, G, g, S, arena, lds_mem, premin, cnt, hs, nodes, donated, words,
-                                  sec);
+                    dfs<V, false>(kp, G, g, S, arena, lds_mem, premin, cnt, hs, nodes, pruned, donated,
+                                  words, sec);
                     if (lane() == 0 && cnt) {
                         atomicAdd(&kp.results[2 * g], cnt);
                         atomicAdd(&kp.results[2 * g + 1], hs);
@@ -2393,7 +2396,7 @@ __global__ __launch_bounds__(64) void mbe_persistent(KParams kp) {
     sec.mark(kSecWait);
     if (idle && lane() == 0) atomicAdd(kp.dq + 2, ~0ull);
     if (lane() == 0) {
-        atomicAdd(&kp.stats[kStatNodes], nodes);
+        atomicAdd(&kp.stats[kStatNodes], nodes - (kp.twins ? pruned : 0));
         atomicAdd(&kp.stats[kStatRoots], roots);
         atomicAdd(&kp.stats[kStatDonated], donated);
         atomicAdd(&kp.stats[kStatStolen], stolen);
@@ -2411,6 +2414,8 @@ __global__ __launch_bounds__(64) void mbe_persistent(KParams kp) {
         }
     }
 }
+
+#include "mbe_tree.h"
 
 // Fill n words with v (clears control words inside captured graphs, where a
 // memset node is not used).
@@ -2453,6 +2458,13 @@ hipError_t launch_put_graph(DevGraph* dst, const DevGraph& g, hipStream_t stream
 // workgroups on `stream`.
 hipError_t launch_mbe(const KParams& kp, uint32_t workers, hipStream_t stream) {
     const size_t lds_bytes = (size_t)kp.lds_words * sizeof(u64);
+    if (kp.tree) {
+        if (kp.sections)
+            hipLaunchKernelGGL(mbe_tree<true>, dim3(workers), dim3(64), lds_bytes, stream, kp);
+        else
+            hipLaunchKernelGGL(mbe_tree<false>, dim3(workers), dim3(64), lds_bytes, stream, kp);
+        return hipGetLastError();
+    }
     switch (kp.variant) {
         case kNoRS:
             hipLaunchKernelGGL(mbe_persistent<kNoRS>, dim3(workers), dim3(64), lds_bytes, stream, kp);
@@ -2486,17 +2498,14 @@ hipError_t launch_fill(unsigned long long* p, uint64_t n, unsigned long long v, 
 
 hipError_t set_lds_limit(uint32_t lds_words) {
     const int bytes = (int)(lds_words * sizeof(u64));
-    hipError_t e = hipFuncSetAttribute((const void*)mbe_persistent<kCuMBE>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)mbe_persistent<kNoRS>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e != hipSuccess) return e;
-    e = hipFuncSetAttribute((const void*)mbe_persistent<kNoES>,
-                            hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    if (e != hipSuccess) return e;
-    return hipFuncSetAttribute((const void*)mbe_persistent<kNoWS>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    const void* kernels[] = {(const void*)mbe_persistent<kCuMBE>, (const void*)mbe_persistent<kNoRS>,
+                             (const void*)mbe_persistent<kNoES>, (const void*)mbe_persistent<kNoWS>,
+                             (const void*)mbe_tree<false>, (const void*)mbe_tree<true>};
+    for (const void* k : kernels) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 #endif  // MBE_EMULATE
 

@@ -77,7 +77,8 @@ struct Ring {
 // candidate with the kept-Q list that localisation builds at the arena's
 // tail, with the distance-two candidate count bounded by the sum of the
 // root's neighbours' other edges.
-uint64_t root_bound_words(const mbe::Prepared& p) {
+// tree: the same for the tree engine's layout.
+uint64_t root_bound_words(const mbe::Prepared& p, uint64_t& tree) {
     std::vector<uint32_t> degL(p.nL);
     for (uint32_t u = 0; u < p.nL; u++) degL[u] = p.offL[u + 1] - p.offL[u];
     uint64_t best = 0;
@@ -93,6 +94,7 @@ uint64_t root_bound_words(const mbe::Prepared& p) {
         const uint64_t lists = (d + 2) / 2 + std::max<uint64_t>(d, (nc + 1) / 2) + 1;
         const uint64_t tail = nc * W + (nc + 1) / 2 + 1;
         best = std::max(best, lists + data + scratch + frames + tail);
+        tree = std::max(tree, mbe::tree_root_words(d, nc));
     }
     return best;
 }
@@ -144,8 +146,8 @@ struct mbe_server {
         m.ng = cfg.table_cap;
         m.max_nr = cfg.max_nr;
         m.total_tasks = 1u << 20;  // overflow-list capacity
-        mbe_status s = setup_pass(b, stream, abort_flag, m, tu, 0, {}, 0, tu.arena_words,
-                                  tu.workers, kp);
+        mbe_status s = setup_pass(b, stream, abort_flag, m, tu, 0, true, {}, 0,
+                                  tu.arena_words, tu.workers, kp);
         if (s != MBE_OK) return s;
         kp.graphs = gtable.as<mbe::DevGraph>();
         kp.n_graphs = 0;
@@ -471,12 +473,13 @@ mbe_status mbe_server_submit(mbe_server* S, const mbe_graph* g, mbe_variant vari
     // footprint: the packed CSR plus the worst-case stack, i.e. the largest
     // local problem (bit matrices and frame stack) one of its roots can build;
     // the per-worker arenas that hold those stacks are allocated once
-    const uint64_t bound = root_bound_words(r->prep);
+    uint64_t tree_bound = 0;
+    const uint64_t bound = root_bound_words(r->prep, tree_bound);
     r->footprint = packed_bytes(r->prep) + bound * 8;
     r->words = packed_bytes(r->prep) / 8;
     // the kernel serves one variant (cuMBE); requests for another variant,
     // or too big for its arenas and tables, take the engine path
-    r->oversize = bound > S->tu.arena_words || r->prep.nR > S->cfg.max_nr ||
+    r->oversize = std::max(bound, tree_bound) > S->tu.arena_words || r->prep.nR > S->cfg.max_nr ||
                   r->words * 8 > S->cfg.data_bytes / 4 || r->words * 8 > S->cfg.staging_bytes / 4 ||
                   variant != MBE_CUMBE;
     if (r->oversize) {

@@ -53,6 +53,7 @@ struct Opt {
 
 template <int V>
 static void wave_fn(void* p) { mbe_persistent<V>(*(KParams*)p); }
+static void tree_fn(void* p) { mbe_tree<false>(*(KParams*)p); }
 
 // Words of the emulated LDS past the launch's dynamic LDS hold this pattern
 // while a wave runs; a write beyond the budget changes one and is reported.
@@ -66,6 +67,7 @@ static uint32_t g_progress_s = 0;
 static void run_pass(KParams& kp, uint32_t workers) {
     void (*fn)(void*) = kp.variant == 1 ? wave_fn<1> : kp.variant == 2 ? wave_fn<2>
                       : kp.variant == 3 ? wave_fn<3> : wave_fn<0>;
+    if (kp.tree) fn = tree_fn;
     std::atomic<bool> pass_done{false};
     std::thread mon;
     if (g_progress_s && kp.progress)
@@ -131,6 +133,16 @@ static void* dalloc(size_t bytes) {
     return p;
 }
 
+// The tree engine's control block and slots (host engine: setup_pass).
+static void tree_setup(KParams& kp, uint32_t workers, bool on) {
+    kp.tree = on;
+    if (!on) return;
+    kp.tworkers = workers;
+    kp.tctl = (unsigned long long*)zalloc((size_t)tree_ctl_words(workers) * 8);
+    kp.tslot_words = std::min<uint64_t>(std::max<uint64_t>(1024, kp.arena_words), 1u << 16);
+    kp.tslots = (uint64_t*)dalloc(kp.tslot_words * workers * 8);
+}
+
 static size_t up_slot(size_t n) { return (n + 8 + 255) & ~(size_t)255; }
 
 // The serving kernel over a list of requests, mirroring the server's device
@@ -183,7 +195,7 @@ static int serve_main(const Opt& o, int n, char** specs) {
     unsigned long long* rem = (unsigned long long*)dalloc((size_t)cap * 32);
     DevGraph* gtable = (DevGraph*)dalloc(cap * sizeof(DevGraph));
     ServeCtl* sctl = (ServeCtl*)zalloc(sizeof(ServeCtl));
-    const uint64_t mark_words = (max_nr + 63) / 64 + 1, cpos_len = max_nr + 1;
+    const uint64_t mark_words = (max_nr + 255) / 256 * 4, cpos_len = max_nr + 1;
     const size_t ctl_words = 2 + kStatCount + kSecCount + 2 * (size_t)cap;
     unsigned long long* ctl = (unsigned long long*)zalloc(ctl_words * 8);
     unsigned long long* dq = (unsigned long long*)zalloc((4 + o.slots) * 8);
@@ -234,6 +246,7 @@ static int serve_main(const Opt& o, int n, char** specs) {
     kp.data = data;
     kp.close = flags + 2;
     kp.done = done;
+    tree_setup(kp, workers, o.twins);
     std::thread host([&] {
         for (int r = 0; r < n; r++) {
             if (o.gap_us) std::this_thread::sleep_for(std::chrono::microseconds(o.gap_us));
@@ -348,7 +361,7 @@ int main(int argc, char** argv) {
     const uint64_t end = o.re ? std::min<uint64_t>(o.re, p.n_roots) : p.n_roots;
     for (uint64_t r = o.rb; r < end; r += o.rs ? o.rs : 1) tasks.push_back(r);
 
-    const uint64_t mark_words = (p.nR + 63) / 64 + 1, cpos_len = (uint64_t)p.nR + 1;
+    const uint64_t mark_words = ((uint64_t)p.nR + 255) / 256 * 4 + 4, cpos_len = (uint64_t)p.nR + 1;
     const size_t ctl_words = 2 + kStatCount + kSecCount + 2;
     unsigned long long* ctl = (unsigned long long*)zalloc(ctl_words * 8);
     unsigned long long* dq = (unsigned long long*)zalloc((4 + o.slots) * 8);
@@ -401,7 +414,10 @@ int main(int argc, char** argv) {
         kp.donate_interval = o.interval;
         kp.dq = dq;
         kp.progress = progress;
+        tree_setup(kp, workers, o.twins && !launches);
         run_pass(kp, workers);
+        free(kp.tctl);
+        free(kp.tslots);
         launches++;
         const uint64_t novf = ctl[1];
         std::vector<uint64_t> next(ovf, ovf + novf);

@@ -1,0 +1,77 @@
+"""The tree engine at the edges of its tiers: levels just inside and just
+outside a tile (64 candidates in P, 128 in Q, rows of 1, 2, 4, 8 and more
+words), wide levels, and hand-over between workers, against the oracle -- on
+the CPU under the wave64 emulator and, marked gpu, on the device.
+
+The graphs are windows: row i is adjacent to the columns i*s .. i*s + d - 1;
+a few rows in the middle have a hole. All rows have about the same degree, so a row's P are the
+windows before it and its Q those after it, up to d / s of each.
+"""
+import os
+import re
+import subprocess
+
+import pytest
+
+import oracle_lib as O
+from graphs import csr_from_edges
+
+M = pytest.importorskip("cumbe_amd")
+EMU_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "emu")
+
+# (rows, window, step, rows with a hole): P up to window / step - 1 and as many Q
+CASES = [
+    (9, 1, 1, 0), (70, 63, 1, 0), (140, 64, 1, 3), (140, 65, 1, 3), (140, 66, 1, 3),
+    (170, 67, 1, 4), (180, 129, 1, 0), (180, 130, 1, 2), (40, 128, 8, 4), (40, 129, 4, 4),
+    (90, 256, 4, 2), (90, 257, 4, 2), (40, 512, 16, 4), (40, 513, 16, 4), (24, 1100, 64, 4),
+]
+
+
+def windows(n, d, s, holes):
+    gone = {n // 2 + i: i * s + d // 2 - i for i in range(holes)}
+    edges = [(i, i * s + j) for i in range(n) for j in range(d) if gone.get(i) != j]
+    return csr_from_edges(n, (n - 1) * s + d, edges)
+
+
+def case_id(c):
+    return "-".join(map(str, c))
+
+
+@pytest.fixture(scope="module")
+def emu():
+    subprocess.run(["make", "-C", EMU_DIR], check=True, capture_output=True)
+
+    def run(path, *opts):
+        out = subprocess.run([os.path.join(EMU_DIR, "emu_run"), *map(str, opts), "bi", path],
+                             capture_output=True, text=True, timeout=300)
+        assert out.returncode == 0, out.stderr
+        m = re.search(r"count (\d+) hash (0x[0-9a-f]+) nodes (\d+) donated (\d+) stolen (\d+)",
+                      out.stdout)
+        return [int(x, 0) for x in m.groups()]
+    return run
+
+
+@pytest.mark.parametrize("case", CASES, ids=case_id)
+def test_tiles_emulated(case, emu, tmp_path):
+    """Default budget; frames and rows in the arena (no LDS room) with
+    hand-over at every step."""
+    g = windows(*case)
+    ref = O.solve(*g)
+    path = str(tmp_path / "w.bi")
+    M.Graph.from_csr(*g).write_bi(path)
+    for opts in (("-w", 4), ("-w", 8, "-l", 420, "-i", 1, "-S", 0)):
+        count, h, nodes, donated, stolen = emu(path, *opts)
+        assert (count, h) == (ref.count, ref.hash), opts
+        assert donated == stolen and nodes >= count
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES, ids=case_id)
+def test_tiles_on_gpu(case):
+    g = windows(*case)
+    ref = O.solve(*g)
+    gg = M.Graph.from_csr(*g)
+    for t in ({}, {"side": 0, "workers": 24, "donate_interval": 1}, {"side": 0, "lds_words": 420}):
+        print(f"windows {case} tuning {t}", flush=True)
+        r = M.solve(gg, "cuMBE", t or None)
+        assert (r.count, r.hash) == (ref.count, ref.hash), t
