@@ -63,7 +63,7 @@ SAMPLE_1CORE = dict(begin=1040, end=0, stride=64)
 LARGE = (200000, 100000, 1500000, 2.0, 2.0, 128)
 LARGE_SEEDS = (11, 12)
 TUNING_KEY = "c1_roots400"
-TUNING = dict(lds_words=3072, waves_per_cu=6, donate_interval=64)
+TUNING = dict(lds_words=2560, waves_per_cu=8, donate_interval=32)
 
 
 def note(msg):

@@ -38,12 +38,12 @@ OCCUPANCY = [(6144, 3), (5120, 4), (4096, 4), (3328, 6), (3072, 6), (2560, 8), (
              (1536, 13)]
 GRID = {
     "occupancy": OCCUPANCY,
-    "donate_interval": [16, 64, 256, 1024],
+    "donate_interval": [16, 32, 64, 256],
     "list_cutoff": [0, 16, 64, 256],
     "compact_ratio": [2, 4, 0xFFFFFFFF],
     "sparse_ratio": [8, 32, 0xFFFFFFFF],
 }
-START = {"occupancy": (3072, 6), "donate_interval": 64, "list_cutoff": 0, "compact_ratio": 2,
+START = {"occupancy": (2560, 8), "donate_interval": 32, "list_cutoff": 0, "compact_ratio": 2,
          "sparse_ratio": 0xFFFFFFFF}
 
 

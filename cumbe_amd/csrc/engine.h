@@ -75,11 +75,11 @@ constexpr uint32_t tree_ctl_words(uint32_t workers) {
 }
 
 // Arena words that a wide level of the tree engine can take: W words of L, nc
-// candidates, np of them in P or X (tile stack, hash terms, reduction scratch,
+// candidates, np of them in P or X (tile memory, hash terms, reduction scratch,
 // rows, frames; nothing in LDS).
 constexpr uint64_t tree_wide_words(uint64_t W, uint64_t nc, uint64_t np) {
     const uint64_t wc = (nc + 63) / 64;
-    return 66 * 13 + 64 * W * 3 + nc + wc * 64 * W + (nc + 1) / 2 + (np + 2) * (4 + W + 3 * wc);
+    return 1632 + 64 * W * 3 + nc + wc * 64 * W + (nc + 1) / 2 + (np + 2) * (4 + W + 3 * wc);
 }
 // and a root of degree d with nc candidates: its candidate lists and rows too
 constexpr uint64_t tree_root_words(uint64_t d, uint64_t nc) {

@@ -2459,10 +2459,12 @@ hipError_t launch_put_graph(DevGraph* dst, const DevGraph& g, hipStream_t stream
 hipError_t launch_mbe(const KParams& kp, uint32_t workers, hipStream_t stream) {
     const size_t lds_bytes = (size_t)kp.lds_words * sizeof(u64);
     if (kp.tree) {
-        if (kp.sections)
-            hipLaunchKernelGGL(mbe_tree<true>, dim3(workers), dim3(64), lds_bytes, stream, kp);
+        if (kp.emit_pos)
+            hipLaunchKernelGGL((mbe_tree<true, true>), dim3(workers), dim3(64), lds_bytes, stream, kp);
+        else if (kp.sections)
+            hipLaunchKernelGGL((mbe_tree<true, false>), dim3(workers), dim3(64), lds_bytes, stream, kp);
         else
-            hipLaunchKernelGGL(mbe_tree<false>, dim3(workers), dim3(64), lds_bytes, stream, kp);
+            hipLaunchKernelGGL((mbe_tree<false, false>), dim3(workers), dim3(64), lds_bytes, stream, kp);
         return hipGetLastError();
     }
     switch (kp.variant) {
@@ -2500,7 +2502,8 @@ hipError_t set_lds_limit(uint32_t lds_words) {
     const int bytes = (int)(lds_words * sizeof(u64));
     const void* kernels[] = {(const void*)mbe_persistent<kCuMBE>, (const void*)mbe_persistent<kNoRS>,
                              (const void*)mbe_persistent<kNoES>, (const void*)mbe_persistent<kNoWS>,
-                             (const void*)mbe_tree<false>, (const void*)mbe_tree<true>};
+                             (const void*)mbe_tree<false, false>,
+                             (const void*)mbe_tree<true, false>, (const void*)mbe_tree<true, true>};
     for (const void* k : kernels) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
         if (e != hipSuccess) return e;

@@ -20,30 +20,58 @@
 //    two per lane; L of at most 8 words. All rows are in VGPRs, all sets are
 //    64-bit scalars, and a node reads no memory: x is a scalar bit scan, L' a
 //    lane read, and the check, absorption, P' and pruning are lane-parallel
-//    compares whose ballots are the new sets. Frames go to a small stack on a
-//    descent only.
+//    compares whose ballots are the new sets. Frames are pushed on a descent
+//    only, into registers too: frame f is lane f of the stack's registers.
 
 constexpr uint32_t kTileP = 64;       // P and X candidates of a tile (lanes)
 constexpr uint32_t kTileQ = 128;      // Q candidates of a tile (two per lane)
 constexpr uint32_t kTileW = 8;        // words of L in a tile
-constexpr uint32_t kTileDepth = 66;   // frames: every descent shrinks P
 constexpr uint32_t kTreeList = 0;     // LDS header: u32[192] gathered candidates
 constexpr uint32_t kTreeHdr = 96;     // LDS words of the header
 static_assert(kTreeHdr <= kLdsSec, "the section counters lie behind the header");
 
-// frame words of a tile of W words: L, P, X, D, R hash sum, |R| and x
+// Narrowing: below a vertex whose L' has at most 64 bits, a tile of more
+// words goes on as a tile of one word over the bits of L', when P' holds at
+// least kNarrowP candidates (gathering the bits takes about two microseconds).
+// The narrow problem's memory: hash terms of the 64 bits and of the lanes,
+// the lanes' rows and the Q rows, its own list.
+constexpr uint32_t kNarrowP = 4;
+constexpr uint32_t kNarrowWords = 64 + 64 + kTileP + kTileQ + (kTileP + kTileQ) / 2;
+
+// frame words of a tile of W words: L, P, X, D, R hash sum, |R| and x. Frame
+// f of a suspended tile is word f of each of these blocks of 64. A pushed
+// frame keeps a candidate in P or is the last, and every descent takes one
+// from P, so 64 frames are enough.
 __device__ __forceinline__ constexpr uint32_t tile_fw(uint32_t W) { return W + 5; }
-static_assert(kTileDepth * tile_fw(kTileW) == 66 * 13 && kTileQ == 2 * 64, "see tree_wide_words");
+__device__ __forceinline__ constexpr uint32_t save_words(uint32_t W) { return 64 * tile_fw(W); }
+static_assert(save_words(1) + save_words(kTileW) + kNarrowWords == 1632 && kTileQ == 2 * 64,
+              "see tree_wide_words");
 // the tile classes: 1, 2, 4 or 8 words
 __device__ __forceinline__ uint32_t tile_class(uint32_t W) {
     return W <= 1 ? 1 : W <= 2 ? 2 : W <= 4 ? 4 : 8;
 }
+
+// This wave's lane numbers, as a function's own: `const Here lane;` hides
+// lane() in it. The compiler takes them as new at that point, so it computes
+// addresses and masks from them there and not before the kernel's loop, where
+// they would fill the registers of every tile search (384 VGPRs with them, 252
+// without, and so one wave per SIMD instead of two).
+struct Here {
+    uint32_t v = lane();
+    __device__ __forceinline__ Here() {
+#ifdef __HIP_DEVICE_COMPILE__
+        asm volatile("" : "+v"(v));
+#endif
+    }
+    __device__ __forceinline__ uint32_t operator()() const { return v; }
+};
 
 __device__ __forceinline__ uint32_t wrlane32(uint32_t old, uint32_t v, uint32_t l) {
     return lane() == l ? v : old;
 }
 __device__ __forceinline__ u64 wrlane64(u64 old, u64 v, uint32_t l) { return lane() == l ? v : old; }
 __device__ __forceinline__ uint32_t uni32(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ bool uni1(bool v) { return uni32(v) != 0; }
 __device__ __forceinline__ u64 low_bits(uint32_t n) { return n >= 64 ? ~0ull : (1ull << n) - 1; }
 
 // Relaxed device-scope accesses: words of another worker's slot and of the
@@ -77,7 +105,9 @@ struct Walk {
     u64 steps;       // vertices taken (the watchdog's and the donation's clock)
     u64 next_event;  // steps at which donation and the watchdog are looked at
     u64 charged;     // steps charged against the node budget
-    uint32_t g;
+    u64 idle;        // lane i: idle workers of the i-th map word looked at
+    uint32_t look;   // the first map word looked at
+    uint32_t g, give;  // give: levels to give away at this event
     bool r_is_u, stop;
 };
 
@@ -89,8 +119,11 @@ __device__ __forceinline__ uint32_t event_interval(const KParams& kp) {
 }
 
 // Watchdog: charge the steps since the last look, look at the abort flag.
+// Every worker looks at the same line, so without a node budget it does every
+// 1,024 steps (some 100 us) and not at every event: with 2,048 workers that
+// took a batch of 64 graphs under a time limit from 16 ms to 23.
 __device__ __forceinline__ void watch(const KParams& kp, Walk& k) {
-    if (!kp.abort) return;
+    if (!kp.abort || (!kp.node_budget && k.steps - k.charged < 1024)) return;
     if (charge_nodes(kp, k.steps - k.charged)) k.stop = true;
     k.charged = k.steps;
 }
@@ -100,12 +133,14 @@ __device__ __forceinline__ void watch(const KParams& kp, Walk& k) {
 // idle map and watches its own flag word; a donor clears the bit (the one
 // whose clear finds it set has the worker), writes the worker's slot and
 // raises the flag. Nothing shared is polled: the flag has a line of its own,
-// the map is read by busy workers once per event and only while the count of
-// active workers is short. (A shared ring that idle workers probe cost its
-// users microseconds per access: the planted background took 15 ms with it
-// and 4 ms with donation off.)
-// Control block (u64 words, 16 to a 128-byte line): [0] active workers, [1]
-// idle ones, [16 (1 + i)] idle map word i, then one flag line per worker: 0
+// and a busy worker looks at a few words of the map once per event, each on a
+// line of its own. (A shared ring that idle workers probe cost its users
+// microseconds per access: the planted background took 15 ms with it and 4 ms
+// with donation off. One count of idle workers that all read was the next
+// limit: with 2,048 workers a batch of 64 graphs took 8.3 ms, and 4.5 with this
+// map.)
+// Control block (u64 words, 16 to a 128-byte line): [0] active workers,
+// [16 (1 + i)] idle map word i, then one flag line per worker: 0
 // none, 1 a level lies in the slot, 2 leave. A worker counts from its start
 // on: the launch may hold more workers than are resident at once, and those
 // that start late find the roots claimed and leave.
@@ -121,34 +156,48 @@ __device__ __forceinline__ unsigned long long* flag_of(const KParams& kp, uint32
 __device__ __forceinline__ u64* slot_of(const KParams& kp, uint32_t w) {
     return (u64*)kp.tslots + (size_t)w * kp.tslot_words;
 }
-__device__ __forceinline__ bool some_idle(const KParams& kp) {
-    return uni64(lane() == 0 ? ld_rlx(kp.tctl + 1) : 0) != 0;
+// Look for idle workers at an event, in kLook words of the map from one that
+// changes from event to event, and say how many levels may go to them: with
+// few idle among many busy, most workers stay out of the race for them (about
+// one donor per idle worker and interval: a claim that fails is an atomic
+// lost); with many idle, more than one.
+constexpr uint32_t kLook = 4, kMaxGive = 2;
+__device__ __forceinline__ uint32_t map_words(const KParams& kp) { return (kp.tworkers + 63) / 64; }
+__device__ __forceinline__ uint32_t may_give(const KParams& kp, Walk& k) {
+    const Here lane;
+    const uint32_t nw = map_words(kp), n = min(nw, kLook);
+    const uint32_t h = (blockIdx.x * 0x9E3779B1u + (uint32_t)k.steps * 0x85EBCA6Bu) >> 8;
+    k.look = h % nw;
+    k.idle = lane() < n ? ld_rlx(idle_word(kp, (k.look + lane()) % nw)) : 0;
+    if (!__ballot(k.idle != 0)) return 0;
+    const uint32_t found = red_add32(__popcll(k.idle));
+    return (h >> 6) % (64 * n) < found ? min(found, kMaxGive) : 0;
 }
-// Claim an idle worker for a level of graph g (its open tasks and the active
-// count are raised first); its number, or ~0.
-__device__ __forceinline__ uint32_t claim_idle(const KParams& kp, uint32_t g) {
-    const uint32_t nw = min((kp.tworkers + 63) / 64, 64u);
-    const uint32_t at = (blockIdx.x + lane()) % nw;  // a start of its own per donor
-    const u64 v = lane() < nw ? ld_rlx(idle_word(kp, at)) : 0;
-    u64 m = __ballot(v != 0);
-    for (uint32_t tries = 0; m && tries < 4; tries++) {
+// Claim one of the idle workers seen, for a level of graph g; its number, or
+// ~0. Whoever clears the worker's bit has it; this donor is active meanwhile,
+// so counting the worker as active can follow.
+__device__ __forceinline__ uint32_t claim_idle(const KParams& kp, Walk& k) {
+    const Here lane;
+    const uint32_t nw = map_words(kp), rot = (blockIdx.x * 0x9E3779B1u) >> 26;
+    for (uint32_t tries = 0; tries < 4; tries++) {
+        const u64 m = __ballot(k.idle != 0);
+        if (!m) break;
         const uint32_t l = __builtin_ctzll(m);
-        const uint32_t wi = rdlane32(at, l);
-        const uint32_t bit = __builtin_ctzll(rdlane64(v, l));
+        const uint32_t wi = (k.look + l) % nw;
+        const u64 v = rdlane64(k.idle, l), up = v >> rot << rot;
+        const uint32_t bit = __builtin_ctzll(up ? up : v);
         u64 old = 0;
-        if (lane() == 0) {
-            atomicAdd(kp.tctl, 1ull);
-            old = atomicAnd(idle_word(kp, wi), ~(1ull << bit));
-            if (!((old >> bit) & 1)) atomicAdd(kp.tctl, ~0ull);
-        }
-        if ((uni64(old) >> bit) & 1) {
+        if (lane() == 0) old = atomicAnd(idle_word(kp, wi), ~(1ull << bit));
+        old = uni64(old);
+        // the word as it is now, without the worker tried
+        k.idle = wrlane64(k.idle, old & ~(1ull << bit), l);
+        if ((old >> bit) & 1) {
             if (lane() == 0) {
-                atomicAdd(kp.tctl + 1, ~0ull);
-                if (kp.remaining) atomicAdd(kp.remaining + 2 * (size_t)g, 1ull);
+                atomicAdd(kp.tctl, 1ull);
+                if (kp.remaining) atomicAdd(kp.remaining + 2 * (size_t)k.g, 1ull);
             }
             return wi * 64 + bit;
         }
-        m &= m - 1;
     }
     return 0xFFFFFFFFu;
 }
@@ -184,12 +233,25 @@ __device__ __forceinline__ LdsSpan lds_span(const KParams& kp, u64* lds) {
     return {lds + (kp.sections ? kLdsHdr : kTreeHdr), lds + kp.lds_words};
 }
 
+// What a tile needs besides its source: where its frames go while it is
+// suspended and, above one word, the narrow problem and that one's frames.
+struct TileMem {
+    u64 *save, *nar, *nsave;
+};
+// n words of LDS, when it has them and `spare` more, else of the arena
+__device__ __forceinline__ u64* place(u64*& lp, const u64* lend, u64*& ap, size_t n, size_t spare) {
+    u64*& at = n + spare <= (size_t)(lend - lp) ? lp : ap;
+    u64* r = at;
+    at += n;
+    return r;
+}
+
 // Place a wide problem (W words, nc candidates of which np in P or X) from
-// arena word off: the tile stack, then the data and the reduction scratch,
+// arena word off: the tile's memory, then the data and the reduction scratch,
 // each in LDS when it fits, then as many frames as LDS holds.
 __device__ __forceinline__ bool layout_wide(const KParams& kp, Wide& S, u64* arena, LdsSpan sp,
                                             size_t off, uint32_t W, uint32_t nc, uint32_t np,
-                                            u64*& tstack) {
+                                            TileMem& M) {
     S.W = W;
     S.nc = nc;
     S.Wc = (nc + 63) >> 6;
@@ -198,22 +260,16 @@ __device__ __forceinline__ bool layout_wide(const KParams& kp, Wide& S, u64* are
     S.maxdepth = np + 2;
     u64* lp = sp.begin;
     u64* ap = arena + off;
-    auto room = [&](size_t n) { return n <= (size_t)(sp.end - lp); };
-    const uint32_t ts = kTileDepth * tile_fw(tile_class(W));
-    u64** at = room(ts) ? &lp : &ap;
-    tstack = *at;
-    *at += ts;
-    const size_t data = (size_t)64 * W + nc + (size_t)S.ncs * W;
-    at = room(data + 2 * S.fs) ? &lp : &ap;
-    S.hl = *at;
+    const uint32_t C = tile_class(W);
+    M.nar = M.nsave = nullptr;
+    if (C > 1) M.nar = place(lp, sp.end, ap, kNarrowWords, 0);
+    S.hl = place(lp, sp.end, ap, (size_t)64 * W + nc + (size_t)S.ncs * W, 2 * S.fs);
     S.hc = S.hl + (size_t)64 * W;
     S.rows = S.hc + nc;
-    *at += data;
-    const size_t scr = (size_t)64 * W * kWideKw + (nc + 1) / 2;
-    at = room(scr + 2 * S.fs) ? &lp : &ap;
-    S.kcols = *at;
+    S.kcols = place(lp, sp.end, ap, (size_t)64 * W * kWideKw + (nc + 1) / 2, 2 * S.fs);
     S.clist = (uint32_t*)(S.kcols + (size_t)64 * W * kWideKw);
-    *at += scr;
+    M.save = place(lp, sp.end, ap, save_words(C), 4 * S.fs);
+    if (C > 1) M.nsave = place(lp, sp.end, ap, save_words(1), 4 * S.fs);
     S.nlds = (uint32_t)min((size_t)S.maxdepth, (size_t)(sp.end - lp) / S.fs);
     S.fbase = lp;
     S.hstack = ap;
@@ -224,6 +280,7 @@ __device__ __forceinline__ bool layout_wide(const KParams& kp, Wide& S, u64* are
 
 // Sum of the hash terms of the set bits of L (W words over hl).
 __device__ __forceinline__ u64 sum_bits(const u64* hl, const u64* L, uint32_t W, uint32_t& nl) {
+    const Here lane;
     u64 s = 0;
     uint32_t n = 0;
     for (uint32_t w = 0; w < W; w++) {
@@ -238,6 +295,7 @@ __device__ __forceinline__ u64 sum_bits(const u64* hl, const u64* L, uint32_t W,
 // Materialisation of one biclique (see emit_biclique): room for the record
 // and its head. Returns where the L' terms go, or null past the capacity.
 __device__ __forceinline__ uint64_t* emit_head(const KParams& kp, uint32_t nl, u64 nr, u64 sr) {
+    const Here lane;
     u64 at = 0;
     if (lane() == 0) {
         at = atomicAdd(&kp.emit_pos[0], (u64)nl + 2);
@@ -286,6 +344,7 @@ __device__ __forceinline__ bool inside_cols(const Row& row, uint32_t k, uint32_t
 template <class Row>
 __device__ __forceinline__ uint32_t reduce_rows(const Row& row, uint32_t W, uint32_t* list,
                                                 uint32_t n, u64* kcols, uint32_t kw, uint32_t& nk) {
+    const Here lane;
     for (uint32_t i = lane(); i < 64 * W * kw; i += 64) kcols[i] = 0;
     sync_own();
     uint32_t kept = 0, idx = 0;
@@ -327,6 +386,7 @@ template <class Row>
 __device__ __forceinline__ uint32_t prune_rows(const Row& row, uint32_t W, uint32_t* list,
                                                uint32_t n, const u64* kcols, uint32_t kw,
                                                uint32_t nk) {
+    const Here lane;
     uint32_t left = 0;
     for (uint32_t b = 0; b < n; b += 64) {
         const bool valid = b + lane() < n;
@@ -341,17 +401,17 @@ __device__ __forceinline__ uint32_t prune_rows(const Row& row, uint32_t W, uint3
 
 // ------------------------------------------------------------------ tile
 // The problem a tile is loaded from: rows[k * ks + w * ws], masked by L when
-// it is given, of the candidates in the gathered list (LDS header): np of P
-// and nx of X first, nq of Q from kTileP on. Tile word i is source word
-// (wmap >> 8 i) & 255. hc[cand[k]] (hc[k] without cand) is candidate k's
+// it is given. Lane i's P, X or D candidate is k = list[i] (LDS header), Q
+// candidates (nq of them) are list[kTileP ..]. P, X and D are the sets to
+// start with; D holds handled vertices, which act as Q. Tile word i is source
+// word (wmap >> 8 i) & 255. hc[cand[k]] (hc[k] without cand) is candidate k's
 // hash term.
 struct TileSrc {
     const u64 *rows, *hc, *L, *hl;
     const uint32_t* cand;
     size_t ks, ws;
-    u64 wmap;
-    uint32_t W, np, nx, nq, nr;
-    u64 sr;
+    u64 wmap, P, X, D, sr;
+    uint32_t W, nq, nr;
     __device__ __forceinline__ uint32_t word(uint32_t i) const { return (wmap >> (8 * i)) & 255; }
     __device__ __forceinline__ u64 row(uint32_t k, uint32_t i) const {
         return rows[k * ks + word(i) * ws];
@@ -359,46 +419,68 @@ struct TileSrc {
 };
 
 // How a search returns to run_tree.
-enum Ret : int { kDone = 0, kToTile = 1, kEvent = 2 };
-constexpr uint32_t kNoX = 64;  // x of a suspended tile's newest frame
+enum Ret : int { kDone = 0, kToTile = 1, kEvent = 2, kToNarrow = 3 };
+constexpr uint32_t kNoX = 64;  // x of a frame without one in progress
+
+// An event: the watchdog, and how many levels this worker may give away.
+// Returns whether the search has to stop for it.
+__device__ __forceinline__ bool event(const KParams& kp, Walk& k) {
+    k.next_event = k.steps + event_interval(kp);
+    watch(kp, k);
+    k.give = kp.variant != kNoWS ? uni32(may_give(kp, k)) : 0;
+    return k.stop || k.give;
+}
 
 // Search of a tile problem, from its start or (resume) from the frames that
-// an event left on the stack. Rows: rp (P and X, lane by lane), n0 and n1
-// (the complements of the Q rows; all ones where a lane holds none). D: the
-// lanes of handled vertices, which act as Q.
-template <int W, bool SEC>
+// it left in save, dep of them, for an event or a narrow tile. Rows: rp (P, X
+// and D, lane by lane), n0 and n1 (the complements of the Q rows; all ones
+// where a lane holds none). Frame f is lane f of fr. A frame is pushed only
+// when its level has candidates left, so a chain of last children returns in
+// one step. The vertex test is a loop of its own: it carries P and X alone.
+// nar: the narrow problem's memory (kNarrowWords), or null when this is one.
+template <int W, bool SEC, bool EMIT>
 __device__ __forceinline__ int tile_search(const KParams& kp, Walk& k, const TileSrc& src,
-                                           const uint32_t* list, u64* stack, uint32_t& depth,
-                                           bool resume, Sec& sec) {
+                                           const uint32_t* list, u64* save, uint32_t& dep,
+                                           bool resume, u64* nar, TileSrc& nsrc, Sec& sec) {
     constexpr uint32_t FW = tile_fw(W);
+    // uniform by construction, which the compiler cannot see through generic
+    // loads and the task's loops: without this the sets are lane values
+    uint32_t depth = resume ? uni32(dep) : 0;
     u64 rp[W], n0[W], n1[W], hcv;
     {
-        const uint32_t npx = src.np + src.nx;
-        const uint32_t pk = lane() < npx ? list[lane()] : 0;
+        const Here lane;
+        const bool in = ((src.P | src.X | src.D) >> lane()) & 1;
+        const uint32_t pk = in ? list[lane()] : 0;
         const uint32_t k0 = lane() < src.nq ? list[kTileP + lane()] : 0;
         const uint32_t k1 = lane() + 64 < src.nq ? list[2 * kTileP + lane()] : 0;
-        hcv = lane() < npx ? src.hc[src.cand ? src.cand[pk] : pk] : 0;
+        hcv = in ? src.hc[src.cand ? src.cand[pk] : pk] : 0;
 #pragma unroll
         for (int i = 0; i < W; i++) {
             const bool have = (uint32_t)i < src.W;
             const u64 m = have ? (src.L ? src.L[src.word(i)] : ~0ull) : 0;
-            rp[i] = have && lane() < npx ? src.row(pk, i) & m : 0;
+            rp[i] = have && in ? src.row(pk, i) & m : 0;
             n0[i] = have && lane() < src.nq ? ~src.row(k0, i) : ~0ull;
             n1[i] = have && lane() + 64 < src.nq ? ~src.row(k1, i) : ~0ull;
         }
     }
-    u64 P = low_bits(src.np), X = low_bits(src.np + src.nx) & ~P, D = 0;
-    int ret = kDone;
+    u64 P = uni64(src.P), X = uni64(src.X), D = uni64(src.D);
     u64 L[W];
 #pragma unroll
     for (int i = 0; i < W; i++) L[i] = ~0ull;
-    u64 sr = src.sr;
-    uint32_t nr = src.nr, nrec = 0;
-    const uint32_t nq = src.nq;
-    if (resume)
-        P = 0;  // the newest frame is taken first
-    else
-        depth = 0;
+    u64 sr = uni64(src.sr);
+    uint32_t nr = uni32(src.nr), nrec = 0, steps = 0;
+    uint32_t limit = uni32(k.next_event > k.steps ? (uint32_t)(k.next_event - k.steps) : 0);
+    uint32_t all = 0;  // steps before the last event
+    u64 fr[FW];
+#pragma unroll
+    for (uint32_t i = 0; i < FW; i++) fr[i] = 0;
+    if (resume) {
+        const Here lane;
+#pragma unroll
+        for (uint32_t i = 0; i < FW; i++) fr[i] = save[i * 64 + lane()];
+    }
+    int ret = kDone;
+    if (resume) P = 0;  // the newest frame is taken first
     u64 recl[W], recs = 0;  // reports not hashed yet: lane i holds report i
     uint32_t recn = 0;
 #pragma unroll
@@ -406,6 +488,7 @@ __device__ __forceinline__ int tile_search(const KParams& kp, Walk& k, const Til
 
     // hash the reports: every lane sums the terms of its own L'
     auto flush = [&]() {
+        const Here lane;
         u64 sl = 0;
         uint32_t nl = 0;
 #pragma unroll
@@ -421,95 +504,95 @@ __device__ __forceinline__ int tile_search(const KParams& kp, Walk& k, const Til
         if (lane() < nrec)
             k.hs += k.r_is_u ? biclique_hash(recs, sl, recn, nl) : biclique_hash(sl, recs, nl, recn);
         k.cnt += nrec;
+        k.nodes += nrec;
         nrec = 0;
     };
-
-    // frame `depth`: L, P, X, D, R hash sum, |R| and the x in progress
     auto push = [&](uint32_t x) {
-        u64 v = 0;
 #pragma unroll
-        for (int i = 0; i < W; i++) v = wrlane64(v, L[i], i);
-        v = wrlane64(v, P, W);
-        v = wrlane64(v, X, W + 1);
-        v = wrlane64(v, D, W + 2);
-        v = wrlane64(v, sr, W + 3);
-        v = wrlane64(v, (u64)nr | ((u64)x << 32), W + 4);
-        if (lane() < FW) stack[(size_t)depth * FW + lane()] = v;
-        wsync();
+        for (int i = 0; i < W; i++) fr[i] = wrlane64(fr[i], L[i], depth);
+        fr[W] = wrlane64(fr[W], P, depth);
+        fr[W + 1] = wrlane64(fr[W + 1], X, depth);
+        fr[W + 2] = wrlane64(fr[W + 2], D, depth);
+        fr[W + 3] = wrlane64(fr[W + 3], sr, depth);
+        fr[W + 4] = wrlane64(fr[W + 4], (u64)nr | ((u64)x << 32), depth);
         depth++;
+    };
+    // whether an event is due that the search has to stop for
+    auto due = [&]() {
+        if (steps < limit) return false;
+        k.steps += steps;
+        all += steps;
+        steps = 0;
+        limit = event_interval(kp);
+        return uni1(event(kp, k));
     };
 
     for (;;) {
-        if (P == 0) {
+        // the next vertex that gives a maximal biclique; what it or a Q row
+        // or a handled vertex covers leaves P and X
+        u64 Lp[W], C = 0, T = 0;
+        uint32_t x = kNoX;
+        u64 P0 = P, X0 = X;
+        while (P) {
+            const uint32_t v = __builtin_ctzll(P);
+            u64 z0 = 0, z1 = 0, zc = 0, zt = 0, zd = 0;
+#pragma unroll
+            for (int i = 0; i < W; i++) {
+                Lp[i] = rdlane64(rp[i], v) & L[i];
+                z0 |= Lp[i] & n0[i];
+                z1 |= Lp[i] & n1[i];
+                const u64 t = rp[i] & Lp[i];
+                zt |= t;
+                zc |= t ^ Lp[i];
+                zd |= rp[i] & (L[i] & ~Lp[i]);
+            }
+            C = __ballot(zc == 0);
+            const u64 dead = __ballot(zd == 0);
+            P0 = P;
+            X0 = X;
+            P &= ~dead;
+            X &= ~dead;
+            steps++;
+            if (!(__ballot(z0 == 0) | __ballot(z1 == 0) | (C & D))) {
+                T = __ballot(zt != 0);
+                x = v;
+                break;
+            }
+        }
+        if (SEC) sec.mark(kSecSelect);
+        if (x == kNoX) {
             if (depth == 0) break;
             depth--;  // ascend: the x in progress joins D
-            const u64 v = stack[(size_t)depth * FW + min(lane(), FW - 1)];
 #pragma unroll
-            for (int i = 0; i < W; i++) L[i] = rdlane64(v, i);
-            P = rdlane64(v, W);
-            X = rdlane64(v, W + 1);
-            D = rdlane64(v, W + 2);
-            sr = rdlane64(v, W + 3);
-            const u64 nx = rdlane64(v, W + 4);
+            for (int i = 0; i < W; i++) L[i] = rdlane64(fr[i], depth);
+            P = rdlane64(fr[W], depth);
+            X = rdlane64(fr[W + 1], depth);
+            D = rdlane64(fr[W + 2], depth);
+            sr = rdlane64(fr[W + 3], depth);
+            const u64 nx = rdlane64(fr[W + 4], depth);
             nr = (uint32_t)nx;
             const uint32_t px = (uint32_t)(nx >> 32);
             if (px != kNoX) D |= 1ull << px;
+            if (SEC) sec.mark(kSecLPrime);
+            if (P && due()) {  // suspend: the level becomes a frame again
+                push(kNoX);
+                ret = kEvent;
+                break;
+            }
             continue;
         }
-        if (k.steps >= k.next_event) {  // suspend: the newest level becomes a frame
-            push(kNoX);
-            ret = kEvent;
-            break;
-        }
-        k.steps++;
-        const uint32_t x = __builtin_ctzll(P);
-        u64 Lp[W];
-        u64 z0 = 0, z1 = 0;
-        if (SEC) sec.mark(kSecSelect);
-#pragma unroll
-        for (int i = 0; i < W; i++) {
-            Lp[i] = rdlane64(rp[i], x) & L[i];
-            z0 |= Lp[i] & n0[i];
-            z1 |= Lp[i] & n1[i];
-        }
-        if (SEC) sec.mark(kSecLPrime);
-        k.words += (u64)W * (nq + __popcll(P | X | D));
-        u64 zc = 0, zt = 0, zd = 0;
-#pragma unroll
-        for (int i = 0; i < W; i++) {
-            const u64 t = rp[i] & Lp[i];
-            zt |= t;
-            zc |= t ^ Lp[i];
-            zd |= rp[i] & (L[i] & ~Lp[i]);
-        }
-        const u64 C = __ballot(zc == 0);
-        const u64 dead = __ballot(zd == 0);
-        if (__ballot(z0 == 0 || z1 == 0) | (C & D)) {  // a Q row holds L'
-            P &= ~dead;
-            X &= ~dead;
-            if (SEC) sec.mark(kSecCheck);
-            continue;
-        }
-        k.nodes++;
-        const u64 T = __ballot(zt != 0);
-        const u64 live = P | X;
+        const u64 live = P0 | X0, ab = live & C;  // x among them
         const u64 Pn = live & T & ~C;
-        u64 ab = live & C;  // x among them
+        u64 sr2 = sr + rdlane64(hcv, x);
+        for (u64 m = ab & ~(1ull << x); m; m &= m - 1) sr2 += rdlane64(hcv, __builtin_ctzll(m));
         const uint32_t nr2 = nr + __popcll(ab);
-        u64 sr2 = sr;
-        while (ab) {
-            sr2 += rdlane64(hcv, __builtin_ctzll(ab));
-            ab &= ab - 1;
-        }
-        P &= ~dead;
-        X &= ~dead;
-        if (SEC) sec.mark(kSecExpand);
+        if (SEC) sec.mark(kSecCheck);
 #pragma unroll
         for (int i = 0; i < W; i++) recl[i] = wrlane64(recl[i], Lp[i], nrec);
         recs = wrlane64(recs, sr2, nrec);
         recn = wrlane32(recn, nr2, nrec);
         nrec++;
-        if (kp.emit_pos) {
+        if (EMIT && kp.emit_pos) {
             uint32_t nl = 0, n = 0;
 #pragma unroll
             for (int i = 0; i < W; i++) nl += __popcll(Lp[i]);
@@ -524,15 +607,88 @@ __device__ __forceinline__ int tile_search(const KParams& kp, Walk& k, const Til
             D |= 1ull << x;
             continue;
         }
-        push(x);
+        bool narrow = false;
+        if (W > 1 && (uint32_t)__popcll(Pn) >= kNarrowP) {
+            uint32_t nl = 0;
+#pragma unroll
+            for (int i = 0; i < W; i++) nl += __popcll(Lp[i]);
+            narrow = nl <= 64;
+        }
+        if (P || narrow) push(x);
+        if (narrow) {
+            // the bits of L' become bits 0, 1, ... of one word
+            u64 a = 0, b0 = 0, b1 = 0;
+            uint32_t t = 0;
+            u64* hl = nar;
+            const Here lane;
+#pragma unroll
+            for (int i = 0; i < W; i++) {
+                const u64 m = Lp[i];
+                if ((m >> lane()) & 1)
+                    hl[t + __popcll(m & lanemask_lt())] = src.hl[src.word(i) * 64 + lane()];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const uint32_t r = (uint32_t)(rp[i] >> (32 * h));
+                    const uint32_t q0 = (uint32_t)(n0[i] >> (32 * h));
+                    const uint32_t q1 = (uint32_t)(n1[i] >> (32 * h));
+                    for (uint32_t mm = (uint32_t)(m >> (32 * h)); mm; mm &= mm - 1, t++) {
+                        const uint32_t b = __builtin_ctz(mm);
+                        a |= (u64)((r >> b) & 1) << t;
+                        b0 |= (u64)((q0 >> b) & 1) << t;
+                        b1 |= (u64)((q1 >> b) & 1) << t;
+                    }
+                }
+            }
+            const u64 all = low_bits(t);
+            u64* hc = nar + 64;
+            u64* rows = hc + 64;
+            uint32_t* nl = (uint32_t*)(rows + kTileP + kTileQ);
+            hc[lane()] = hcv;
+            rows[lane()] = a;
+            rows[kTileP + lane()] = ~b0 & all;
+            rows[2 * kTileP + lane()] = ~b1 & all;
+            for (uint32_t q = lane(); q < kTileP + kTileQ; q += 64) nl[q] = q;
+            wsync();
+            nsrc.rows = rows;
+            nsrc.hc = hc;
+            nsrc.L = nullptr;
+            nsrc.hl = hl;
+            nsrc.cand = nullptr;
+            nsrc.ks = nsrc.ws = 1;
+            nsrc.wmap = 0;
+            nsrc.P = Pn;
+            nsrc.X = 0;
+            nsrc.D = D;
+            nsrc.sr = sr2;
+            nsrc.W = 1;
+            nsrc.nq = src.nq;
+            nsrc.nr = nr2;
+            ret = kToNarrow;
+            if (SEC) sec.mark(kSecCompact);
+            break;
+        }
 #pragma unroll
         for (int i = 0; i < W; i++) L[i] = Lp[i];
         P = Pn;
         X = 0;
         sr = sr2;
         nr = nr2;
+        if (SEC) sec.mark(kSecExpand);
+        if (due()) {
+            push(kNoX);
+            ret = kEvent;
+            break;
+        }
     }
     if (nrec) flush();
+    dep = depth;
+    if (ret != kDone) {
+        const Here lane;
+#pragma unroll
+        for (uint32_t i = 0; i < FW; i++) save[i * 64 + lane()] = fr[i];
+    }
+    k.steps += steps;
+    k.words += (u64)(all + steps) * W * (src.nq + __popcll(src.P | src.X | src.D));
     wsync();
     return ret;
 }
@@ -540,6 +696,7 @@ __device__ __forceinline__ int tile_search(const KParams& kp, Walk& k, const Til
 // --------------------------------------------------------------- wide walk
 // Candidates of a bit mask (Wc words), ascending, into list; returns how many.
 __device__ __forceinline__ uint32_t gather_bits(const u64* M, uint32_t Wc, uint32_t* list) {
+    const Here lane;
     uint32_t n = 0;
     for (uint32_t b = 0; b < Wc; b++) {
         const u64 m = uni64(M[b]);
@@ -568,7 +725,8 @@ __device__ __forceinline__ uint32_t word_map(const u64* L, uint32_t W, u64& wmap
 // contain and the P candidates that Q candidates contain.
 __device__ __forceinline__ int place_level(const Wide& S, u64* F, uint32_t pn, uint32_t xn,
                                            uint32_t qn, uint32_t* list, TileSrc& src) {
-    const uint32_t W = S.W, Wc = S.Wc;
+    const Here lane;
+    const uint32_t W = uni32(S.W), Wc = uni32(S.Wc);
     const u64* L = F + kFrameHdr;
     u64* P = F + kFrameHdr + W;
     u64* Q = P + 2 * Wc;
@@ -612,8 +770,9 @@ __device__ __forceinline__ int place_level(const Wide& S, u64* F, uint32_t pn, u
     src.cand = nullptr;
     src.hl = S.hl;
     src.L = L;
-    src.np = pn;
-    src.nx = xn;
+    src.P = low_bits(pn);
+    src.X = low_bits(pn + xn) & ~src.P;
+    src.D = 0;
     src.nq = qn;
     src.sr = uni64(F[1]);
     src.nr = (uint32_t)uni64(F[2]);
@@ -623,11 +782,13 @@ __device__ __forceinline__ int place_level(const Wide& S, u64* F, uint32_t pn, u
 // Walk the wide levels from level k until a child fits the tile (kToTile,
 // src set; its level is k + 1), an event is due (kEvent) or the problem is
 // finished (kDone). resume: level k's x in progress has just been handled.
-template <bool SEC>
+template <bool SEC, bool EMIT>
 __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide& S, uint32_t& k,
                                           bool resume, uint32_t* list, TileSrc& src, Sec& sec) {
-    const uint32_t W = S.W, Wc = S.Wc;
+    const Here lane;
+    const uint32_t W = uni32(S.W), Wc = uni32(S.Wc);
     for (;;) {
+        k = uni32(k);
         u64* F = S.frame(k);
         u64* L = F + kFrameHdr;
         u64* P = L + W;
@@ -641,7 +802,7 @@ __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide
             wsync();
             resume = false;
         }
-        if (wk.steps >= wk.next_event) return kEvent;
+        if (wk.steps >= wk.next_event && uni1(event(kp, wk))) return kEvent;
         // the next x: the lowest candidate left in P
         uint32_t x = 0xFFFFFFFFu;
         for (uint32_t b0 = 0; b0 < Wc && x == 0xFFFFFFFFu; b0 += 64) {
@@ -735,7 +896,7 @@ __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide
         const u64 h = wk.r_is_u ? biclique_hash(sr, sl, nr, nl) : biclique_hash(sl, sr, nl, nr);
         wk.cnt++;
         if (lane() == 0) wk.hs += h;
-        if (kp.emit_pos) {
+        if (EMIT && kp.emit_pos) {
             uint32_t n = 0;
             uint64_t* o = emit_head(kp, nl, nr, sr);
             for (uint32_t w = 0; w < W && o; w++) emit_word(o, n, uni64(Lc[w]), S.hl + w * 64);
@@ -762,10 +923,15 @@ __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide
 }
 
 // -------------------------------------------------------------- donation
-// The upper part of P that a level gives away: all but the lower half.
-__device__ __forceinline__ u64 upper_part(u64 P, uint32_t keep) {
-    for (uint32_t i = 0; i < keep; i++) P &= P - 1;
-    return P;
+// What a level keeps of P when it gives: the first half, of which a level
+// without an x in progress always has one; nothing when it gives the rest.
+__device__ __forceinline__ uint32_t keep_of(uint32_t n, bool rest, bool running) {
+    return running ? (rest ? 0 : n / 2) : max(1u, n / 2);
+}
+__device__ __forceinline__ u64 first_bits(u64 P, uint32_t n) {
+    u64 r = P;
+    for (uint32_t i = 0; i < n; i++) r &= r - 1;
+    return P & ~r;
 }
 __device__ __forceinline__ size_t slot_need(uint32_t W, uint32_t npx, uint32_t nq) {
     return (size_t)kSlotHeaderWords + (size_t)64 * W + npx + (size_t)W * (npx + nq);
@@ -786,12 +952,14 @@ __device__ __forceinline__ void slot_head(u64* slot, uint32_t g, uint32_t W, uin
 }
 
 // Give away part of the shallowest wide level with unselected work: the donor
-// keeps the lower half A of P and moves the rest B to X; the thief gets
-// P = B, X, Q u A u x. The order "x, A, B, X" is a valid order of the level,
-// so both sides report exactly the bicliques of the sequential walk. Levels
-// 1..cur have their x in progress; cur has none when idle_cur is set.
+// keeps the first candidates A of P (keep_of) and moves the rest B to X; the
+// thief gets P = B, X and Q u A u x. The order "x, A, B, X" is a valid order
+// of the level, so both sides report exactly the bicliques of the sequential
+// walk. Levels 1..cur have their x in progress; cur has none when idle_cur is
+// set.
 __device__ __forceinline__ bool donate_wide(const KParams& kp, const Wide& S, uint32_t cur,
-                                            bool idle_cur, uint32_t g) {
+                                            bool idle_cur, bool rest, Walk& wk) {
+    const Here lane;
     const uint32_t W = S.W, Wc = S.Wc;
     const uint32_t top = kp.donate_depth ? min(cur, kp.donate_depth) : cur;
     for (uint32_t k = 1; k <= top; k++) {
@@ -806,21 +974,23 @@ __device__ __forceinline__ bool donate_wide(const KParams& kp, const Wide& S, ui
         const bool running = k < cur || !idle_cur;
         if (pc == 0 || (!running && pc < 2)) continue;
         const uint32_t x = running ? uni32((uint32_t)F[0]) : 0xFFFFFFFFu;
-        const uint32_t keep = pc / 2;
-        // sizes: B, X, and the Q side (Q, A, x); t = first candidate of B
-        uint32_t seen = 0, t = 0xFFFFFFFFu, nx = 0, nq = 0;
+        const uint32_t keep = keep_of(pc, rest, running), np = pc - keep;
+        // sizes, and t = the first candidate of B
+        uint32_t seen = 0, t = keep ? Wc * 64 : 0, nx = 0, nq = keep + (running ? 1 : 0);
         for (uint32_t b = 0; b < Wc; b++) {
             const u64 pw = uni64(P[b]);
-            if (t == 0xFFFFFFFFu && seen + __popcll(pw) > keep)
-                t = b * 64 + __builtin_ctzll(upper_part(pw, keep - seen));
-            seen += __popcll(pw);
+            const uint32_t c = __popcll(pw);
+            if (seen < keep && seen + c >= keep) {
+                const u64 up = pw & ~first_bits(pw, keep - seen);
+                t = b * 64 + (up ? __builtin_ctzll(up) : 64);
+            }
+            seen += c;
             nx += __popcll(uni64(X[b]));
             nq += __popcll(uni64(Q[b]));
         }
-        nq += keep + (running ? 1 : 0);
-        const uint32_t np = pc - keep, npx = np + nx, n = npx + nq;
+        const uint32_t npx = np + nx, n = npx + nq;
         if (!slot_fits(kp, W, npx, nq)) continue;
-        const uint32_t to = claim_idle(kp, g);
+        const uint32_t to = uni32(claim_idle(kp, wk));
         if (to == 0xFFFFFFFFu) return false;
         u64* slot = slot_of(kp, to);
         u64* hl = slot + kSlotHeaderWords;
@@ -829,11 +999,11 @@ __device__ __forceinline__ bool donate_wide(const KParams& kp, const Wide& S, ui
         for (uint32_t i = lane(); i < 64 * W; i += 64) st_rlx(hl + i, S.hl[i]);
         uint32_t ip = 0, ix = np, iq = npx;
         for (uint32_t b = 0; b < Wc; b++) {
-            const u64 pw = uni64(P[b]), xw = uni64(X[b]);
-            const u64 up = b * 64 >= t ? ~0ull : (b * 64 + 64 <= t ? 0ull : ~0ull << (t & 63));
-            u64 qw = uni64(Q[b]) | (pw & ~up);
+            const u64 pw = uni64(P[b]);
+            const u64 aw = b * 64 >= t ? 0 : pw & low_bits(t - b * 64);
+            const u64 bw = pw & ~aw, xw = uni64(X[b]);
+            u64 qw = uni64(Q[b]) | aw;
             if (running && b == (x >> 6)) qw |= 1ull << (x & 63);
-            const u64 bw = pw & up;
             const u64 all = bw | xw | qw;
             const uint32_t kk = b * 64 + lane();
             if ((all >> lane()) & 1) {
@@ -849,13 +1019,13 @@ __device__ __forceinline__ bool donate_wide(const KParams& kp, const Wide& S, ui
             ix += __popcll(xw);
             iq += __popcll(qw);
         }
-        slot_head(slot, g, W, np, nx, nq, F[1], F[2]);
+        slot_head(slot, wk.g, W, np, nx, nq, F[1], F[2]);
         hand_over(kp, to);
         for (uint32_t b = lane(); b < Wc; b += 64) {
-            const u64 up = b * 64 >= t ? ~0ull : (b * 64 + 64 <= t ? 0ull : ~0ull << (t & 63));
             const u64 pw = P[b];
-            X[b] |= pw & up;
-            P[b] = pw & ~up;
+            const u64 aw = b * 64 >= t ? 0 : pw & low_bits(t - b * 64);
+            X[b] |= pw & ~aw;
+            P[b] = aw;
         }
         wsync();
         return true;
@@ -863,28 +1033,28 @@ __device__ __forceinline__ bool donate_wide(const KParams& kp, const Wide& S, ui
     return false;
 }
 
-// The same from the frames of a suspended tile (depth of them; the newest has
-// no x in progress). Rows come from the tile's source; level: how many wide
+// The same from the frames of a suspended tile (depth of them; the newest may
+// have no x in progress). Rows come from the tile's source; level: how many
 // levels lie above.
 __device__ __forceinline__ bool donate_tile(const KParams& kp, const TileSrc& src,
-                                            const uint32_t* list, u64* stack, uint32_t depth,
-                                            uint32_t level, uint32_t g) {
-    const uint32_t W = src.W, C = tile_class(W), FW = tile_fw(C);
+                                            const uint32_t* list, u64* save, uint32_t depth,
+                                            uint32_t level, bool rest, Walk& wk) {
+    const Here lane;
+    const uint32_t W = src.W, C = tile_class(W);
     for (uint32_t f = 0; f < depth; f++) {
         if (kp.donate_depth && level + f + 1 > kp.donate_depth) return false;
-        u64* F = stack + (size_t)f * FW;
-        const u64 P = uni64(F[C]), X = uni64(F[C + 1]);
-        const uint32_t x = (uint32_t)uni32((uint32_t)(F[C + 4] >> 32));
-        if (P == 0 || (x == kNoX && __popcll(P) < 2)) continue;
-        u64 D = uni64(F[C + 2]);
-        if (x != kNoX) D |= 1ull << x;
-        const uint32_t keep = __popcll(P) / 2;
-        const u64 B = upper_part(P, keep);
-        const u64 qp = D | (P & ~B);  // lanes that become Q
+        u64* F = save + f;
+        const u64 P = uni64(F[64 * C]);
+        const uint32_t x = uni32((uint32_t)(F[64 * (C + 4)] >> 32)), pc = __popcll(P);
+        if (P == 0 || (x == kNoX && pc < 2)) continue;
+        const u64 D = uni64(F[64 * (C + 2)]);
+        const u64 A = first_bits(P, keep_of(pc, rest, x != kNoX)), B = P & ~A;
+        const u64 X = uni64(F[64 * (C + 1)]);
+        const u64 qp = (x == kNoX ? D : D | (1ull << x)) | A;  // lanes that become Q
         const uint32_t np = __popcll(B), nx = __popcll(X), npx = np + nx;
         const uint32_t nq = __popcll(qp) + src.nq, n = npx + nq;
         if (!slot_fits(kp, W, npx, nq)) continue;
-        const uint32_t to = claim_idle(kp, g);
+        const uint32_t to = uni32(claim_idle(kp, wk));
         if (to == 0xFFFFFFFFu) return false;
         u64* slot = slot_of(kp, to);
         u64* hl = slot + kSlotHeaderWords;
@@ -899,18 +1069,18 @@ __device__ __forceinline__ bool donate_tile(const KParams& kp, const TileSrc& sr
         const uint32_t q0 = npx + __popcll(qp);
         if (have && at < npx) st_rlx(hc + at, src.hc[src.cand ? src.cand[pk] : pk]);
         for (uint32_t i = 0; i < W; i++) {
-            const u64 L = F[i] & (src.L ? src.L[src.word(i)] : ~0ull);
+            const u64 L = F[64 * i] & (src.L ? src.L[src.word(i)] : ~0ull);
             u64* r = rows + (size_t)i * n;
             st_rlx(hl + i * 64 + lane(), src.hl[src.word(i) * 64 + lane()]);
             if (have) st_rlx(r + at, src.row(pk, i) & L);
             for (uint32_t q = lane(); q < src.nq; q += 64)
                 st_rlx(r + q0 + q, src.row(list[kTileP + q], i) & L);
         }
-        slot_head(slot, g, W, np, nx, nq, uni64(F[C + 3]), (uint32_t)uni64(F[C + 4]));
+        slot_head(slot, wk.g, W, np, nx, nq, uni64(F[64 * (C + 3)]), (uint32_t)uni64(F[64 * (C + 4)]));
         hand_over(kp, to);
         if (lane() == 0) {
-            F[C] = P & ~B;
-            F[C + 1] = X | B;
+            F[64 * C] = A;
+            F[64 * (C + 1)] = X | B;
         }
         wsync();
         return true;
@@ -919,29 +1089,50 @@ __device__ __forceinline__ bool donate_tile(const KParams& kp, const TileSrc& sr
 }
 
 // ----------------------------------------------------------------- tasks
+// The descriptors, which every lane holds alike, as the scalars they are: the
+// compiler loses track of that where a root and a handed-over level merge, and
+// lane values would cost a vector register each.
+template <class T>
+__device__ __forceinline__ void uni_one(T& v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (sizeof(T) == 8)
+        v = (T)uni64((u64)v);
+    else
+        v = (T)uni32((uint32_t)v);
+#endif
+}
+template <class... T>
+__device__ __forceinline__ void uni_all(T&... v) {
+    (uni_one(v), ...);
+}
+__device__ __forceinline__ void make_uniform(Wide& S) {
+    uni_all(S.W, S.nc, S.Wc, S.ncs, S.fs, S.nlds, S.maxdepth, S.hl, S.hc, S.rows, S.fbase, S.hstack,
+            S.kcols, S.clist);
+}
+__device__ __forceinline__ void make_uniform(TileSrc& s) {
+    uni_all(s.rows, s.hc, s.L, s.hl, s.cand, s.wmap, s.P, s.X, s.D, s.sr, s.ks, s.ws, s.W, s.nq, s.nr);
+}
+__device__ __forceinline__ void make_uniform(Walk& k) {
+    uni_all(k.cnt, k.nodes, k.donated, k.words, k.steps, k.next_event, k.charged, k.look, k.g, k.give,
+            k.r_is_u, k.stop);
+}
+__device__ __forceinline__ void make_uniform(TileMem& M) { uni_all(M.save, M.nar, M.nsave); }
+
 // What a task starts with after localisation or a slot load.
 enum TreeStart : int { kTreeOverflow = -1, kTreeDone = 0, kTreeTile = 1, kTreeWide = 2 };
 
-// Place the tile stack and the 64 W hash terms of a task that starts as a
-// tile, from arena word off; returns the arena words in use.
+// Place the memory and the 64 W hash terms of a task that starts as a tile,
+// from arena word off; returns the arena words in use.
 __device__ __forceinline__ size_t layout_tile(u64* arena, LdsSpan sp, size_t off, uint32_t W,
-                                              u64*& tstack, u64*& hl) {
+                                              TileMem& M, u64*& hl) {
     u64* lp = sp.begin;
     u64* ap = arena + off;
-    const uint32_t ts = kTileDepth * tile_fw(tile_class(W));
-    if (lp + ts <= sp.end) {
-        tstack = lp;
-        lp += ts;
-    } else {
-        tstack = ap;
-        ap += ts;
-    }
-    if (lp + 64 * W <= sp.end) {
-        hl = lp;
-    } else {
-        hl = ap;
-        ap += 64 * W;
-    }
+    const uint32_t C = tile_class(W);
+    M.nar = M.nsave = nullptr;
+    if (C > 1) M.nar = place(lp, sp.end, ap, kNarrowWords, 0);
+    hl = place(lp, sp.end, ap, 64 * W, 0);
+    M.save = place(lp, sp.end, ap, save_words(C), 0);
+    if (C > 1) M.nsave = place(lp, sp.end, ap, save_words(1), 0);
     return (size_t)(ap - arena);
 }
 
@@ -952,6 +1143,7 @@ __device__ __forceinline__ size_t layout_tile(u64* arena, LdsSpan sp, size_t off
 template <class F>
 __device__ __forceinline__ uint32_t for_entries(const DevGraph& G, const uint32_t* Nx, uint32_t d,
                                                 uint32_t* lb, F&& fn) {
+    const Here lane;
     uint32_t total = 0;
     for (uint32_t j0 = 0; j0 < d; j0 += 64) {
         const uint32_t n = min(64u, d - j0);
@@ -1019,17 +1211,19 @@ __device__ __forceinline__ int place_start(const Wide& S, u64* F, uint32_t np, u
 // worker's mark and rank tables and at the arena's tail. A problem that fits
 // the tile is gathered from these rows as they are; any other is laid out by
 // word for the wide tier.
+template <bool EMIT>
 __device__ __forceinline__ int build_tree_root(const KParams& kp, const DevGraph& G, uint32_t x,
                                                u64* arena, u64* lds, u64* gmark, uint32_t* cpos,
-                                               Walk& wk, Wide& S, TileSrc& src, u64*& tstack,
+                                               Walk& wk, Wide& S, TileSrc& src, TileMem& M,
                                                uint32_t* list, u64& build) {
-    const uint32_t s0 = G.offR[x];
+    const Here lane;
+    const uint32_t s0 = uni32(G.offR[x]);
     const uint32_t d = uni32(G.offR[x + 1] - s0);
     const uint32_t* Nx = G.adjR + s0;
     if (d == 0) return kTreeDone;
     const uint32_t W = (d + 63) >> 6;
     LdsSpan sp = lds_span(kp, lds);
-    const uint32_t nblk = (G.nR + 255) >> 8, nwords = nblk * 4;
+    const uint32_t nblk = (uni32(G.nR) + 255) >> 8, nwords = nblk * 4;
     u64* mark = gmark;
     uint32_t* pre = cpos;
     const bool lds_mark = sp.begin + nwords + (nblk + 1) / 2 <= sp.end;
@@ -1065,7 +1259,7 @@ __device__ __forceinline__ int build_tree_root(const KParams& kp, const DevGraph
     off += nc + 1;  // P and Q positions, and the sorted Q
     const size_t row_words = (size_t)nc * W;
     const uint32_t lds_low = max(lds_mark ? nwords + (nblk + 1) / 2 : 0u,
-                                 kTileDepth * tile_fw(tile_class(W)) + 64 * W);
+                                 (W > 1 ? kNarrowWords : 0) + 64 * W);
     const bool lds_rows = row_words + lds_low <= (size_t)(sp.end - sp.begin);
     const size_t tail_words = lds_rows ? 0 : row_words;
     // roots that list mode suits (see build_root) and those whose rows do
@@ -1126,7 +1320,7 @@ __device__ __forceinline__ int build_tree_root(const KParams& kp, const DevGraph
     }
     ab = red_add32(ab);
     abh = red_add64(abh);
-    const u64 sr = G.hR[x] + abh;
+    const u64 sr = uni64(G.hR[x]) + abh;
     const uint32_t nr = 1 + ab;
     uint32_t nq = np ? nc - kx : 0;
     sync_own();
@@ -1182,9 +1376,9 @@ __device__ __forceinline__ int build_tree_root(const KParams& kp, const DevGraph
     u64* hl = arena + off;  // a leaf root's terms, for materialisation
     size_t end = off + (size_t)64 * W;
     if (direct) {
-        end = layout_tile(arena, sp, off, W, tstack, hl);
+        end = layout_tile(arena, sp, off, W, M, hl);
     } else if (np) {
-        if (!layout_wide(kp, S, arena, sp, off, W, np + nq, min(np, d), tstack)) return kTreeOverflow;
+        if (!layout_wide(kp, S, arena, sp, off, W, np + nq, min(np, d), M)) return kTreeOverflow;
         hl = S.hl;
         end = S.end;
     }
@@ -1203,7 +1397,7 @@ __device__ __forceinline__ int build_tree_root(const KParams& kp, const DevGraph
     const u64 h = wk.r_is_u ? biclique_hash(sr, sl, nr, d) : biclique_hash(sl, sr, d, nr);
     if (lane() == 0) wk.hs += h;
     sync_own();
-    if (kp.emit_pos) {
+    if (EMIT && kp.emit_pos) {
         uint64_t* o = emit_head(kp, d, nr, sr);
         if (o)
             for (uint32_t j = lane(); j < d; j += 64) o[j] = hl[j];
@@ -1222,8 +1416,8 @@ __device__ __forceinline__ int build_tree_root(const KParams& kp, const DevGraph
         src.L = nullptr;
         src.wmap = 0x0706050403020100ull;
         src.W = W;
-        src.np = np;
-        src.nx = 0;
+        src.P = low_bits(np);
+        src.X = src.D = 0;
         src.nq = nq;
         src.sr = sr;
         src.nr = nr;
@@ -1260,8 +1454,9 @@ __device__ __forceinline__ int build_tree_root(const KParams& kp, const DevGraph
 // Copy a donated level out of the worker's slot: a tile as it is, or a wide
 // problem, which is tried as a tile once more.
 __device__ __forceinline__ int load_tree_slot(const KParams& kp, u64* slot, u64* arena,
-                                              u64* lds, Wide& S, TileSrc& src, u64*& tstack,
+                                              u64* lds, Wide& S, TileSrc& src, TileMem& M,
                                               uint32_t* list) {
+    const Here lane;
     const u64 s1 = uni64(ld_rlx(slot + 1)), s2 = uni64(ld_rlx(slot + 2));
     const uint32_t W = (uint32_t)s1, np = (uint32_t)(s1 >> 32);
     const uint32_t nx = (uint32_t)s2, nq = (uint32_t)(s2 >> 32);
@@ -1271,7 +1466,7 @@ __device__ __forceinline__ int load_tree_slot(const KParams& kp, u64* slot, u64*
     u64* rows0 = hc0 + npx;
     if (npx <= kTileP && nq <= kTileQ && W <= kTileW) {
         u64* hl;
-        const size_t off = layout_tile(arena, lds_span(kp, lds), kArenaHdr, W, tstack, hl);
+        const size_t off = layout_tile(arena, lds_span(kp, lds), kArenaHdr, W, M, hl);
         u64* rows = arena + off;
         u64* hc = rows + (size_t)W * n;
         if (off + (size_t)W * n + npx > kp.arena_words) return kTreeOverflow;
@@ -1290,14 +1485,15 @@ __device__ __forceinline__ int load_tree_slot(const KParams& kp, u64* slot, u64*
         src.L = nullptr;
         src.wmap = 0x0706050403020100ull;
         src.W = W;
-        src.np = np;
-        src.nx = nx;
+        src.P = low_bits(np);
+        src.X = low_bits(npx) & ~src.P;
+        src.D = 0;
         src.nq = nq;
         src.sr = uni64(ld_rlx(slot + 3));
         src.nr = (uint32_t)uni64(ld_rlx(slot + 4));
         return kTreeTile;
     }
-    if (!layout_wide(kp, S, arena, lds_span(kp, lds), kArenaHdr, W, n, min(npx, 64 * W), tstack)) return kTreeOverflow;
+    if (!layout_wide(kp, S, arena, lds_span(kp, lds), kArenaHdr, W, n, min(npx, 64 * W), M)) return kTreeOverflow;
     for (uint32_t i = lane(); i < 64 * W; i += 64) S.hl[i] = ld_rlx(hl0 + i);
     for (uint32_t k = lane(); k < S.ncs; k += 64) {
         if (k < n) S.hc[k] = k < npx ? ld_rlx(hc0 + k) : 0;
@@ -1323,42 +1519,74 @@ __device__ __forceinline__ int load_tree_slot(const KParams& kp, u64* slot, u64*
     return place_start(S, F1, np, nx, nq, list, src);
 }
 
-// Run a task from its start to its end.
-template <bool SEC>
+// Run a task from its start to its end: the wide walk, the tile it leads to,
+// and the narrow tile that one leads to, whichever is current.
+template <bool SEC, bool EMIT>
 __device__ __forceinline__ void run_tree(const KParams& kp, Walk& wk, int start, const Wide& S,
-                                         TileSrc& src, u64* tstack, uint32_t* list, Sec& sec) {
-    const bool wide = start == kTreeWide;
-    uint32_t k = wide ? 1 : 0, depth = 0;
-    bool tile = !wide, resume = false;  // resume: of a tile, or of level k after its x
+                                         TileSrc& src, const TileMem& M, uint32_t* list,
+                                         Sec& sec) {
+    enum { kWideWalk, kTile, kNarrow };
+    const bool wide = uni1(start == kTreeWide);
+    uint32_t k = wide ? 1 : 0, depth = 0, ndepth = 0;
+    int at = wide ? kWideWalk : kTile;
+    bool resume = false;  // of a tile, or of level k after its x
+    TileSrc nsrc{};
     for (;;) {
         int r;
-        if (!tile)
-            r = wide_walk<SEC>(kp, wk, S, k, resume, list, src, sec);
-        else
-            switch (tile_class(src.W)) {
-                case 1: r = tile_search<1, SEC>(kp, wk, src, list, tstack, depth, resume, sec); break;
-                case 2: r = tile_search<2, SEC>(kp, wk, src, list, tstack, depth, resume, sec); break;
-                case 4: r = tile_search<4, SEC>(kp, wk, src, list, tstack, depth, resume, sec); break;
-                default: r = tile_search<8, SEC>(kp, wk, src, list, tstack, depth, resume, sec); break;
-            }
+        at = (int)uni32(at);
+        k = uni32(k);
+        depth = uni32(depth);
+        ndepth = uni32(ndepth);
+        resume = uni1(resume);
+        make_uniform(wk);
+        make_uniform(src);
+        make_uniform(nsrc);
+        const uint32_t cls = at == kTile ? tile_class(uni32(src.W)) : at == kNarrow ? 1 : 0;
+        if (cls == 0) {
+            r = wide_walk<SEC, EMIT>(kp, wk, S, k, resume, list, src, sec);
+        } else if (cls == 1) {
+            const bool n = at == kNarrow;
+            TileSrc none;
+            r = tile_search<1, SEC, EMIT>(
+                kp, wk, n ? nsrc : src, n ? (uint32_t*)(nsrc.rows + kTileP + kTileQ) : list,
+                n ? M.nsave : M.save, n ? ndepth : depth, resume, nullptr, none, sec);
+        } else if (cls == 2) {
+            r = tile_search<2, SEC, EMIT>(kp, wk, src, list, M.save, depth, resume, M.nar, nsrc, sec);
+        } else if (cls == 4) {
+            r = tile_search<4, SEC, EMIT>(kp, wk, src, list, M.save, depth, resume, M.nar, nsrc, sec);
+        } else {
+            r = tile_search<8, SEC, EMIT>(kp, wk, src, list, M.save, depth, resume, M.nar, nsrc, sec);
+        }
+        r = (int)uni32(r);
+        make_uniform(wk);
         if (r == kEvent) {
-            wk.next_event = wk.steps + event_interval(kp);
-            watch(kp, wk);
             if (wk.stop) return;
             if (SEC) sec.mark(kSecOther);
-            if (kp.variant != kNoWS && some_idle(kp)) {
-                // the level above a tile has its x in progress
-                bool gave = wide && donate_wide(kp, S, k, !tile, wk.g);
-                if (!gave && tile) gave = donate_tile(kp, src, list, tstack, depth, k, wk.g);
+            // half of the shallowest level with work left, then the rest of it
+            bool rest = false;
+            for (bool gave = true; wk.give && gave; wk.give--, rest = !rest) {
+                // the levels above the current tier have their x in progress
+                gave = wide && uni1(donate_wide(kp, S, k, at == kWideWalk, rest, wk));
+                if (!gave && at != kWideWalk)
+                    gave = uni1(donate_tile(kp, src, list, M.save, depth, k, rest, wk));
+                if (!gave && at == kNarrow)
+                    gave = uni1(donate_tile(kp, nsrc, (uint32_t*)(nsrc.rows + kTileP + kTileQ),
+                                            M.nsave, ndepth, k + depth, rest, wk));
                 wk.donated += gave;
                 if (SEC) sec.mark(kSecDonate);
             }
-            resume = tile;
+            resume = at != kWideWalk;
         } else if (r == kToTile) {
-            tile = true;
+            at = kTile;
             resume = false;
-        } else if (tile && wide) {
-            tile = false;
+        } else if (r == kToNarrow) {
+            at = kNarrow;
+            resume = false;
+        } else if (at == kNarrow) {
+            at = kTile;
+            resume = true;
+        } else if (at == kTile && wide) {
+            at = kWideWalk;
             resume = true;
         } else {
             return;
@@ -1371,6 +1599,7 @@ __device__ __forceinline__ void run_tree(const KParams& kp, Walk& wk, int start,
 // as active before it takes a root, so that no other worker leaves meanwhile.
 __device__ __forceinline__ bool claim_served(const KParams& kp, uint32_t wid, bool idle, uint32_t& g,
                                              uint32_t& x) {
+    const Here lane;
     u64 got = 0, gg = 0, xx = 0;
     if (lane() == 0) {
         ServeCtl* sc = kp.serve;
@@ -1407,8 +1636,8 @@ __device__ __forceinline__ bool claim_served(const KParams& kp, uint32_t wid, bo
 // One worker of the tree engine: roots first, then levels handed over by
 // other workers; it leaves when every worker is idle (served kernels: once
 // the host has closed the mailbox, too).
-template <bool SEC>
-__global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
+template <bool SEC, bool EMIT>
+__global__ __launch_bounds__(64, 2) void mbe_tree(KParams kp) {
     extern __shared__ u64 lds_mem[];
     const uint32_t wid = blockIdx.x;
     u64* arena = (u64*)kp.arena + (size_t)wid * kp.arena_words;
@@ -1416,9 +1645,8 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
     uint32_t* cpos = kp.cpos + (size_t)wid * kp.cpos_len;
     uint32_t* list = (uint32_t*)(lds_mem + kTreeList);
     Sec sec;
-    sec.init(SEC, lds_mem);
+    sec.init(SEC && kp.sections, lds_mem);
     Walk wk{};
-    wk.next_event = event_interval(kp);
     u64 roots = 0, ovf = 0, stolen = 0, dropped = 0, build = 0;
     bool roots_left = true, idle = false;
     uint32_t backoff = 1;
@@ -1426,17 +1654,19 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
     if (lane() == 0) atomicAdd(kp.tctl, 1ull);
     for (;;) {
         wsync();
-        const bool stop = aborted(kp);
+        const bool stop = uni1(aborted(kp));
         if (stop) roots_left = false;
-        Wide S;
-        TileSrc src;
-        u64* tstack = nullptr;
+        Wide S{};
+        TileSrc src{};
+        TileMem M{};
         int start = kTreeDone;
         uint32_t x = 0;
         bool got = false, failed = false;
         u64 task = 0;
         wk.cnt = wk.hs = 0;
         wk.stop = false;
+        // a task of less than an interval is not worth splitting
+        wk.next_event = wk.steps + event_interval(kp);
         if (roots_left) {
             u64 t = 0;
             if (kp.serve) {
@@ -1461,9 +1691,7 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
                 u64 old = 0;
                 if (lane() == 0) old = atomicAnd(idle_word(kp, wid >> 6), ~my_bit);
                 idle = false;
-                if (uni64(old) & my_bit) {
-                    if (lane() == 0) atomicAdd(kp.tctl + 1, ~0ull);
-                } else {
+                if (!(uni64(old) & my_bit)) {
                     // its level comes after this root; the donor counted this
                     // worker as active a second time
                     if (lane() == 0) atomicAdd(kp.tctl, ~0ull);
@@ -1479,7 +1707,7 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
                 if (SEC) sec.mark(kSecWait);
                 u64* slot = slot_of(kp, wid);
                 wk.g = (uint32_t)uni64(ld_rlx(slot));
-                start = stop ? kTreeOverflow : load_tree_slot(kp, slot, arena, lds_mem, S, src, tstack, list);
+                start = stop ? kTreeOverflow : load_tree_slot(kp, slot, arena, lds_mem, S, src, M, list);
                 failed = start < 0;
                 dropped += failed && !stop;
                 stolen++;
@@ -1491,13 +1719,13 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
         if (got) {
             backoff = 1;
             const DevGraph G = kp.graphs[wk.g];
-            wk.r_is_u = G.r_is_u;
+            wk.r_is_u = uni1(G.r_is_u);
             if (x != 0xFFFFFFFFu) {
-                if (kp.serve) task = G.task_base + x;
-                else x = (uint32_t)(task - G.task_base);
+                if (kp.serve) task = uni64(G.task_base) + x;
+                else x = (uint32_t)(task - uni64(G.task_base));
                 if (SEC) sec.mark(kSecOther);
-                start = build_tree_root(kp, G, x, arena, lds_mem, mark, cpos, wk, S, src, tstack,
-                                        list, build);
+                start = build_tree_root<EMIT>(kp, G, x, arena, lds_mem, mark, cpos, wk, S, src,
+                                              M, list, build);
                 if (SEC) sec.mark(kSecBuild);
                 if (start < 0) {
                     ovf++;
@@ -1510,7 +1738,10 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
                     roots++;
                 }
             }
-            if (start > 0) run_tree<SEC>(kp, wk, start, S, src, tstack, list, sec);
+            start = (int)uni32(start);
+            make_uniform(S);
+            make_uniform(M);
+            if (start > 0) run_tree<SEC, EMIT>(kp, wk, start, S, src, M, list, sec);
             if (kp.node_budget) watch(kp, wk);
             const u64 hs = red_add64(wk.hs);
             if (lane() == 0 && wk.cnt) {
@@ -1530,7 +1761,7 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
             }
             continue;
         }
-        if (kp.serve && !stop && serve_load(kp)) {
+        if (kp.serve && !stop && uni1(serve_load(kp))) {
             backoff = 1;
             continue;
         }
@@ -1540,7 +1771,6 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
             idle = true;
             u64 left = 0;
             if (lane() == 0) {
-                atomicAdd(kp.tctl + 1, 1ull);
                 atomicOr(idle_word(kp, wid >> 6), my_bit);
                 left = atomicAdd(kp.tctl, ~0ull) - 1;
             }
@@ -1549,23 +1779,29 @@ __global__ __launch_bounds__(64) void mbe_tree(KParams kp) {
                 break;
             }
         } else if (kp.serve) {
-            if (serve_exit(kp, uni64(lane() == 0 ? ld_rlx(kp.tctl) : 0), stop)) break;
+            if (uni1(serve_exit(kp, uni64(lane() == 0 ? ld_rlx(kp.tctl) : 0), stop))) break;
         }
-        for (uint32_t i = 0; i < backoff; i++) __builtin_amdgcn_s_sleep(8);
+        // served workers look at the mailbox ever less often, all of them at
+        // the same lines; each watches its own flag all the while, or every
+        // level handed over would first lie there for some 50 us
+        for (uint32_t i = 0; i < backoff; i++) {
+            __builtin_amdgcn_s_sleep(8);
+            if (kp.serve && (i & 3) == 3 && uni64(lane() == 0 ? ld_rlx(flag_of(kp, wid)) : 0)) break;
+        }
         backoff = min(backoff * 2, kp.serve ? 256u : 4u);
         if (SEC) sec.mark(kSecWait);
     }
     if (SEC) sec.mark(kSecWait);
     if (lane() == 0) {
-        atomicAdd(&kp.stats[kStatNodes], wk.nodes);
-        atomicAdd(&kp.stats[kStatRoots], roots);
-        atomicAdd(&kp.stats[kStatDonated], wk.donated);
-        atomicAdd(&kp.stats[kStatStolen], stolen);
-        atomicAdd(&kp.stats[kStatOverflow], ovf);
-        atomicAdd(&kp.stats[kStatBuildWords], build);
-        atomicAdd(&kp.stats[kStatDropped], dropped);
-        atomicAdd(&kp.stats[kStatWords], wk.words);
-        if (SEC)
+        // a worker that found no task has nothing to add
+        const u64 st[][2] = {{kStatNodes, wk.nodes},       {kStatRoots, roots},
+                             {kStatDonated, wk.donated},   {kStatStolen, stolen},
+                             {kStatOverflow, ovf},         {kStatBuildWords, build},
+                             {kStatDropped, dropped},      {kStatWords, wk.words}};
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            if (st[i][1]) atomicAdd(&kp.stats[st[i][0]], st[i][1]);
+        if (SEC && kp.sections)
             for (int i = 0; i < kSecCount; i++) atomicAdd(&kp.sections[i], sec.t[i]);
         if (SEC && kp.worker_busy) {
             u64 busy = 0;

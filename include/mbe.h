@@ -66,7 +66,7 @@ typedef struct {
     uint32_t compact_ratio;  /* re-localise a child subproblem when its universe
                                 shrank by this factor; 0 = default (2),
                                 UINT32_MAX = never */
-    uint32_t donate_interval;/* nodes between a worker's donation checks; 0 = 64 */
+    uint32_t donate_interval;/* nodes between a worker's donation checks; 0 = 32 */
     int32_t side;            /* -1 reference side choice, 0 enumerate U, 1 V */
     uint32_t flags;          /* MBE_FLAG_* */
     /* Root subset: ranks r with root_begin <= r < root_end (0 = all) and

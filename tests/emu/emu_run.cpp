@@ -53,7 +53,7 @@ struct Opt {
 
 template <int V>
 static void wave_fn(void* p) { mbe_persistent<V>(*(KParams*)p); }
-static void tree_fn(void* p) { mbe_tree<false>(*(KParams*)p); }
+static void tree_fn(void* p) { mbe_tree<false, false>(*(KParams*)p); }
 
 // Words of the emulated LDS past the launch's dynamic LDS hold this pattern
 // while a wave runs; a write beyond the budget changes one and is reported.
