@@ -41,6 +41,10 @@ double now_ms();
         }                                                                                  \
     } while (0)
 
+// Free the device buffers that a destroyed server left for the next one (see
+// serve.cpp); whether there were any.
+bool give_back_kept();
+
 // Device buffer that grows on demand and is reused across solves.
 struct DevBuf {
     void* p = nullptr;
@@ -51,6 +55,10 @@ struct DevBuf {
         p = nullptr;
         bytes = 0;
         hipError_t e = hipMalloc(&p, need);
+        if (e == hipErrorOutOfMemory && give_back_kept()) {
+            (void)hipGetLastError();
+            e = hipMalloc(&p, need);
+        }
         if (e == hipSuccess) bytes = need;
         return e;
     }
@@ -73,6 +81,13 @@ struct Bufs {
                                      hipHostMallocMapped | hipHostMallocCoherent);
         if (e == hipSuccess) progress_slots = 2 * workers;
         return e;
+    }
+    size_t device_bytes() const {
+        size_t n = 0;
+        for (const DevBuf* b : {&arena, &mark, &cpos, &ctl, &graphs, &data, &ovf, &slots, &dq, &busy,
+                                &tctl, &tslots})
+            n += b->bytes;
+        return n;
     }
     void release() {
         for (DevBuf* b : {&arena, &mark, &cpos, &ctl, &graphs, &data, &ovf, &slots, &dq, &busy, &tctl,

@@ -16,6 +16,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <unistd.h>
 
 #include "host.h"
@@ -23,6 +24,39 @@
 namespace {
 
 using namespace mbe::host;
+
+// The launch buffers of the last server destroyed, for the next one: at the
+// default launch 9.4 GB, mostly arenas. The driver wipes freed memory before
+// it gives it out again, so a program that creates a server per burst waited
+// 250 ms in every destroy once it had been through the card's memory (some 30
+// servers); the burst itself takes 14. One set is kept at most, and none above
+// 16 GiB; an allocation of this library that fails gives it back, unless a
+// server is alive: its kernel runs on, and a free would wait for that.
+constexpr size_t kKeepBytes = (size_t)16 << 30;
+struct Kept {
+    std::mutex m;
+    Bufs b;
+    int servers = 0;
+};
+Kept& kept() {
+    static Kept* k = new Kept();  // never destroyed: outlives HIP teardown
+    return *k;
+}
+// The kept set, for a new server (servers: 1) or to be freed (0).
+Bufs take_kept(int servers) {
+    std::lock_guard<std::mutex> lk(kept().m);
+    if (!servers && kept().servers) return Bufs{};
+    kept().servers += servers;
+    return std::exchange(kept().b, Bufs{});
+}
+// b's work has ended. Its buffers are kept, or else the ones kept before.
+void keep(Bufs& b) {
+    if (b.device_bytes() <= kKeepBytes) {
+        std::lock_guard<std::mutex> lk(kept().m);
+        if (b.device_bytes() > kept().b.device_bytes()) std::swap(b, kept().b);
+    }
+    b.release();
+}
 
 struct Req {
     uint64_t id = 0;
@@ -381,11 +415,22 @@ struct mbe_server {
     }
 };
 
+namespace mbe::host {
+bool give_back_kept() {
+    Bufs b = take_kept(0);
+    const bool any = b.device_bytes() != 0;
+    b.release();
+    return any;
+}
+}  // namespace mbe::host
+
 namespace {
 
 void free_server(mbe_server* S) {
-    if (S->stream) (void)hipStreamSynchronize(S->stream);
-    S->b.release();
+    if (S->stream && hipStreamSynchronize(S->stream) == hipSuccess && !S->failed)
+        keep(S->b);
+    else
+        S->b.release();
     for (DevBuf* d : {&S->gtable, &S->rem, &S->sctl, &S->data}) {
         if (d->p) (void)hipFree(d->p);
         d->p = nullptr;
@@ -395,9 +440,12 @@ void free_server(mbe_server* S) {
         if (h) (void)hipHostFree(h);
     if (S->ev_end) (void)hipEventDestroy(S->ev_end);
     if (S->stream) (void)hipStreamDestroy(S->stream);
+    std::lock_guard<std::mutex> lk(kept().m);
+    kept().servers--;
 }
 
 mbe_status make_server(mbe_server* S) {
+    S->b = take_kept(1);
     HIPC(hipSetDevice(0));
     hipDeviceProp_t prop;
     HIPC(hipGetDeviceProperties(&prop, 0));
