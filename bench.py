@@ -339,8 +339,8 @@ def main():
             "traffic": traffic,
             "traffic_GBps": traffic / launch_s / 1e9 if traffic else None,
             "algorithmic_bytes_per_launch": op_bytes,
-            "limiter": ("latency of dependent LDS and L2 accesses (three single-wave workers "
-                        "per CU, LDS-limited); the operand words are served mostly from LDS"),
+            "limiter": ("issue and latency of one wave's chain of vertex tests (two waves per "
+                        "SIMD, register-limited); the operand words are served from registers"),
             "launch_ms": launch_ms,
             "reference_equivalent_GBps": ref_gbps,
             "reference_work_entries": w_alg,

@@ -1,4 +1,8 @@
-// gfx950 kernels of the MBE engine.
+// gfx950 kernels of the MBE engine: the general engine, and (mbe_tree.h) the
+// tree engine, which runs the first pass of every call unless the reference's
+// tree is asked for. The general engine takes that tree, and the roots that
+// the tree engine leaves to a later pass. What follows describes the general
+// engine.
 //
 // Execution model: a persistent grid of single-wave workgroups; each wave64
 // is one worker (the reference's "block", src/mbe_noWS.cuh:101-615). A

@@ -39,9 +39,10 @@ constexpr uint32_t kNarrowP = 4;
 constexpr uint32_t kNarrowWords = 64 + 64 + kTileP + kTileQ + (kTileP + kTileQ) / 2;
 
 // frame words of a tile of W words: L, P, X, D, R hash sum, |R| and x. Frame
-// f of a suspended tile is word f of each of these blocks of 64. A pushed
-// frame keeps a candidate in P or is the last, and every descent takes one
-// from P, so 64 frames are enough.
+// f of a suspended tile is word f of each of these blocks of 64. Every descent
+// takes at least x from the at most 64 candidates of P and X together, and a
+// level is pushed only while it or its child has some in P, so 64 frames are
+// enough.
 __device__ __forceinline__ constexpr uint32_t tile_fw(uint32_t W) { return W + 5; }
 __device__ __forceinline__ constexpr uint32_t save_words(uint32_t W) { return 64 * tile_fw(W); }
 static_assert(save_words(1) + save_words(kTileW) + kNarrowWords == 1632 && kTileQ == 2 * 64,
@@ -1633,6 +1634,10 @@ __device__ __forceinline__ bool claim_served(const KParams& kp, uint32_t wid, bo
     return got != 0;
 }
 
+// What bounds the kernel is one wave's chain of dependent vertex tests, so the
+// registers are kept to what two waves per SIMD allow (256). A batch of 256
+// graphs: 33.7 ms with 377 registers and one wave, 17.4 with two; bounds of
+// three or four waves spill and were slower.
 // One worker of the tree engine: roots first, then levels handed over by
 // other workers; it leaves when every worker is idle (served kernels: once
 // the host has closed the mailbox, too).
