@@ -144,7 +144,10 @@ __device__ __forceinline__ void watch(const KParams& kp, Walk& k) {
 // [16 (1 + i)] idle map word i, then one flag line per worker: 0
 // none, 1 a level lies in the slot, 2 leave. A worker counts from its start
 // on: the launch may hold more workers than are resident at once, and those
-// that start late find the roots claimed and leave.
+// that start late find the roots claimed and leave. It waits for its count to
+// be performed before it claims a root: then whoever finds the roots claimed
+// and the count at zero knows that nobody works, and that no level will be
+// handed to the workers it sends away.
 // Slot: [0] graph, [1] W | np << 32, [2] nx | nq << 32, [3] R hash sum,
 // [4] |R|, then hl[64 W], hc[np + nx], the rows of P, X and Q by word
 // (W x (np + nx + nq)).
@@ -1614,7 +1617,10 @@ __device__ __forceinline__ bool claim_served(const KParams& kp, uint32_t wid, bo
                 if (f >= la) break;
                 const uint32_t gl = kp.lane_list[(size_t)ln * kp.mail_cap + f];
                 const u64 n = kp.graphs[gl].n_roots;
-                if (idle) atomicAdd(kp.tctl, 1ull);
+                if (idle) {
+                    atomicAdd(kp.tctl, 1ull);
+                    __builtin_amdgcn_s_waitcnt(0);
+                }
                 const u64 c = atomicAdd(&kp.root_cursor[gl], 1ull);
                 if (c < n) {
                     got = 1;
@@ -1657,6 +1663,7 @@ __global__ __launch_bounds__(64, 2) void mbe_tree(KParams kp) {
     uint32_t backoff = 1;
     const u64 my_bit = 1ull << (wid & 63);
     if (lane() == 0) atomicAdd(kp.tctl, 1ull);
+    wait_mem();
     for (;;) {
         wsync();
         const bool stop = uni1(aborted(kp));
@@ -1677,7 +1684,7 @@ __global__ __launch_bounds__(64, 2) void mbe_tree(KParams kp) {
             if (kp.serve) {
                 got = claim_served(kp, wid, idle, wk.g, x);
             } else {
-                t = uni64(lane() == 0 ? atomicAdd(kp.cursor, 1ull) : 0);
+                t = uni64(lane() == 0 ? (u64)atomicAdd(kp.cursor, 1ull) : 0);
                 got = t < kp.n_tasks;
                 roots_left = got;
             }
@@ -1797,6 +1804,9 @@ __global__ __launch_bounds__(64, 2) void mbe_tree(KParams kp) {
         if (SEC) sec.mark(kSecWait);
     }
     if (SEC) sec.mark(kSecWait);
+    // nothing is handed to a worker that has left (under a watchdog others may
+    // still be at work)
+    if (idle && lane() == 0) atomicAnd(idle_word(kp, wid >> 6), ~my_bit);
     if (lane() == 0) {
         // a worker that found no task has nothing to add
         const u64 st[][2] = {{kStatNodes, wk.nodes},       {kStatRoots, roots},

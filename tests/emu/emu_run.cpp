@@ -21,6 +21,8 @@
 //          -L large_edges (serve: requests with at least this many edges take
 //             the large claim lane) -T table_cap (serve) -u publish gap (us)
 //          -G seed of the garbage that fills uncleared device buffers
+//          -D us: a late atomic (wave_emu.h) lingers up to us after the next
+//             one, by a random sequence of seed -G
 //          -P s: print the workers' progress every s seconds (stderr)
 #include "wave_emu.h"
 #include "../../cumbe_amd/csrc/mbe_kernel.hip"
@@ -319,7 +321,8 @@ int main(int argc, char** argv) {
             case 'L': o.large_edges = (uint32_t)v; break;
             case 'T': o.table_cap = (uint32_t)v; break;
             case 'u': o.gap_us = (uint32_t)v; break;
-            case 'G': g_fill_seed = (uint64_t)v; break;
+            case 'G': g_fill_seed = emu::g_linger_seed = (uint64_t)v; break;
+            case 'D': emu::g_linger_us = (uint32_t)v; break;
             case 'P': g_progress_s = (uint32_t)v; break;
             default: fprintf(stderr, "unknown option -%c\n", f); return 2;
         }

@@ -11,9 +11,16 @@
 // a divergent cross-lane operation. Waves run on separate OS threads, so
 // global atomics and the work-stealing deque see real concurrency. LDS is
 // a thread_local array per wave.
+//
+// Nothing but a wait orders an atomic whose result is not used with the wave's
+// next one on another address, so it is performed late here: when the wave
+// waits (s_waitcnt, a fence, a release store), sleeps or touches the address
+// again, or after the next atomic that does return. There the wave first
+// lingers, up to g_linger_us at random, so that others see the later one alone.
 #pragma once
 #include <sched.h>
 #include <ucontext.h>
+#include <unistd.h>
 
 #include <chrono>
 #include <cstdint>
@@ -21,6 +28,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
+#include <vector>
 
 #define __device__
 #define __global__
@@ -60,6 +68,98 @@ inline thread_local uint32_t g_block = 0, g_grid = 1;
 [[noreturn]] inline void die(const char* what) {
     fprintf(stderr, "wave emulator: %s (block %u)\n", what, g_block);
     abort();
+}
+
+// This wave's late atomics, at most one per address.
+struct Late {
+    void* p;
+    void (*perform)(void*, uint64_t);
+    uint64_t v;
+};
+constexpr size_t kMaxLate = 64;
+inline thread_local std::vector<Late> g_late;
+inline thread_local uint64_t g_rand = 0;
+inline uint32_t g_linger_us = 0;
+inline uint64_t g_linger_seed = 1;
+
+inline void perform_late() {
+    while (!g_late.empty()) {
+        const Late l = g_late.back();
+        g_late.pop_back();
+        l.perform(l.p, l.v);
+    }
+}
+inline void perform_late(const volatile void* p) {
+    for (size_t i = 0; i < g_late.size(); i++)
+        if (g_late[i].p == p) {
+            const Late l = g_late[i];
+            g_late.erase(g_late.begin() + i);
+            l.perform(l.p, l.v);
+            return;
+        }
+}
+inline void linger() {
+    if (g_late.empty()) return;
+    if (g_linger_us) {
+        if (!g_rand) g_rand = g_linger_seed * 0x9E3779B97F4A7C15ull + (g_block + 1) * 0xD6E8FEB86659FD93ull;
+        g_rand ^= g_rand << 13;
+        g_rand ^= g_rand >> 7;
+        g_rand ^= g_rand << 17;
+        usleep((useconds_t)(g_rand % g_linger_us));
+    }
+    perform_late();
+}
+
+// What an atomic returns: performed when that is read, late when it is not.
+template <class T, class Op>
+struct Atomic {
+    T* p;
+    T v;
+    bool read = false;
+    Atomic(T* p_, T v_) : p(p_), v(v_) {}
+    Atomic(const Atomic&) = delete;
+    operator T() {
+        read = true;
+        perform_late(p);
+        const T r = Op::perform(p, v);
+        linger();
+        return r;
+    }
+    ~Atomic() {
+        if (read) return;
+        perform_late(p);
+        if (g_late.size() == kMaxLate) perform_late();
+        g_late.push_back({p, [](void* q, uint64_t w) { Op::perform((T*)q, (T)w); }, (uint64_t)v});
+    }
+};
+struct OpAdd {
+    template <class T>
+    static T perform(T* p, T v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
+};
+struct OpOr {
+    template <class T>
+    static T perform(T* p, T v) { return __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST); }
+};
+struct OpAnd {
+    template <class T>
+    static T perform(T* p, T v) { return __atomic_fetch_and(p, v, __ATOMIC_SEQ_CST); }
+};
+template <class T>
+inline T load(T* p) {
+    perform_late(p);
+    return __atomic_load_n(p, __ATOMIC_SEQ_CST);
+}
+template <class T, class U>
+inline void store(T* p, U v, int order) {
+    if (order == __ATOMIC_RELAXED)
+        perform_late(p);
+    else
+        perform_late();
+    __atomic_store_n(p, (T)v, __ATOMIC_SEQ_CST);
+}
+inline void wait() {
+    perform_late();
+    __atomic_thread_fence(__ATOMIC_SEQ_CST);
 }
 
 inline uint64_t xlane(int op, uint64_t val, uint64_t old = 0, uint64_t arg = 0) {
@@ -176,6 +276,7 @@ inline void run_wave(uint32_t block, uint32_t grid, void (*fn)(void*), void* arg
         }
         for (int l = 0; l < 64; l++) w->state[l] = 0;
     }
+    perform_late();
     g_wave = nullptr;
     free(stacks);
     delete w;
@@ -199,10 +300,13 @@ inline int __builtin_amdgcn_update_dpp(int old, int src, int ctrl, int row_mask,
                            (uint64_t)(ctrl & 0xFFFF) | ((uint64_t)row_mask << 16));
 }
 inline void __syncthreads() { emu::xlane(emu::kBarrier, 0); }
-inline void __threadfence() { __atomic_thread_fence(__ATOMIC_SEQ_CST); }
-inline void __builtin_amdgcn_fence(int, const char*) { __atomic_thread_fence(__ATOMIC_SEQ_CST); }
-inline void __builtin_amdgcn_s_sleep(int) { sched_yield(); }
-inline void __builtin_amdgcn_s_waitcnt(int) {}
+inline void __threadfence() { emu::wait(); }
+inline void __builtin_amdgcn_fence(int, const char*) { emu::wait(); }
+inline void __builtin_amdgcn_s_sleep(int) {
+    emu::wait();
+    sched_yield();
+}
+inline void __builtin_amdgcn_s_waitcnt(int) { emu::wait(); }
 inline unsigned long long wall_clock64() {
     return (unsigned long long)std::chrono::duration_cast<std::chrono::nanoseconds>(
                std::chrono::steady_clock::now().time_since_epoch())
@@ -211,13 +315,14 @@ inline unsigned long long wall_clock64() {
 inline int __popcll(unsigned long long v) { return __builtin_popcountll(v); }
 
 template <class T, class U>
-inline T atomicAdd(T* p, U v) { return __atomic_fetch_add(p, (T)v, __ATOMIC_SEQ_CST); }
+inline emu::Atomic<T, emu::OpAdd> atomicAdd(T* p, U v) { return {p, (T)v}; }
 template <class T, class U>
-inline T atomicOr(T* p, U v) { return __atomic_fetch_or(p, (T)v, __ATOMIC_SEQ_CST); }
+inline emu::Atomic<T, emu::OpOr> atomicOr(T* p, U v) { return {p, (T)v}; }
 template <class T, class U>
-inline T atomicAnd(T* p, U v) { return __atomic_fetch_and(p, (T)v, __ATOMIC_SEQ_CST); }
+inline emu::Atomic<T, emu::OpAnd> atomicAnd(T* p, U v) { return {p, (T)v}; }
 template <class T, class U>
 inline T atomicMax(T* p, U v) {
+    emu::perform_late(p);
     T c = __atomic_load_n(p, __ATOMIC_SEQ_CST);
     while (c < (T)v &&
            !__atomic_compare_exchange_n(p, &c, (T)v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST)) {
@@ -226,14 +331,15 @@ inline T atomicMax(T* p, U v) {
 }
 template <class T, class U, class V>
 inline T atomicCAS(T* p, U cmp, V val) {
+    emu::perform_late(p);
     T c = (T)cmp;
     __atomic_compare_exchange_n(p, &c, (T)val, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);
     return c;
 }
-#define __hip_atomic_load(p, order, scope) __atomic_load_n((p), __ATOMIC_SEQ_CST)
+#define __hip_atomic_load(p, order, scope) emu::load(p)
 #define __hip_atomic_fetch_or(p, v, order, scope) __atomic_fetch_or((p), (v), __ATOMIC_SEQ_CST)
 #define __hip_atomic_fetch_add(p, v, order, scope) __atomic_fetch_add((p), (v), __ATOMIC_SEQ_CST)
-#define __hip_atomic_store(p, v, order, scope) __atomic_store_n((p), (v), __ATOMIC_SEQ_CST)
+#define __hip_atomic_store(p, v, order, scope) emu::store((p), (v), (order))
 
 template <class A, class B>
 inline typename std::common_type<A, B>::type min(A a, B b) {

@@ -41,8 +41,8 @@ def case_id(c):
 def emu():
     subprocess.run(["make", "-C", EMU_DIR], check=True, capture_output=True)
 
-    def run(path, *opts):
-        out = subprocess.run([os.path.join(EMU_DIR, "emu_run"), *map(str, opts), "bi", path],
+    def run(*args):
+        out = subprocess.run([os.path.join(EMU_DIR, "emu_run"), *map(str, args)],
                              capture_output=True, text=True, timeout=300)
         assert out.returncode == 0, out.stderr
         m = re.search(r"count (\d+) hash (0x[0-9a-f]+) nodes (\d+) donated (\d+) stolen (\d+)",
@@ -60,7 +60,7 @@ def test_tiles_emulated(case, emu, tmp_path):
     path = str(tmp_path / "w.bi")
     M.Graph.from_csr(*g).write_bi(path)
     for opts in (("-w", 4), ("-w", 8, "-l", 420, "-i", 1, "-S", 0)):
-        count, h, nodes, donated, stolen = emu(path, *opts)
+        count, h, nodes, donated, stolen = emu(*opts, "bi", path)
         assert (count, h) == (ref.count, ref.hash), opts
         assert donated == stolen and nodes >= count
 
@@ -75,3 +75,20 @@ def test_tiles_on_gpu(case):
         print(f"windows {case} tuning {t}", flush=True)
         r = M.solve(gg, "cuMBE", t or None)
         assert (r.count, r.hash) == (ref.count, ref.hash), t
+
+
+PLANTED = (6500, 1900, 0.008, 60, 8, 40, 0.05, 3)
+
+
+@pytest.mark.parametrize("workers", [2, 4])
+def test_late_count_keeps_idle_workers(workers, emu):
+    """One deep root, and atomics without a result performed up to 20 ms late:
+    a worker that finds no root must not send the others away while the one
+    with the root has not been counted yet. Levels handed to a worker that
+    has left would be missing from the count."""
+    ref = O.solve_roots(*M.Graph.er_planted(*PLANTED).csr(), begin=11, end=12, threads=1)
+    for seed in range(1, 7):
+        count, h, _, donated, stolen = emu("-w", workers, "-i", 1, "-b", 11, "-e", 12, "-D", 20000,
+                                           "-G", seed, "er", *PLANTED)
+        assert (count, h) == (ref.count, ref.hash), seed
+        assert donated == stolen > 0
