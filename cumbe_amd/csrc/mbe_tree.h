@@ -148,9 +148,11 @@ __device__ __forceinline__ void watch(const KParams& kp, Walk& k) {
 // be performed before it claims a root: then whoever finds the roots claimed
 // and the count at zero knows that nobody works, and that no level will be
 // handed to the workers it sends away.
-// Slot: [0] graph, [1] W | np << 32, [2] nx | nq << 32, [3] R hash sum,
+// Slot: [0] graph | r_is_u << 32, [1] W | np << 32, [2] nx | nq << 32, [3] R hash sum,
 // [4] |R|, then hl[64 W], hc[np + nx], the rows of P, X and Q by word
-// (W x (np + nx + nq)).
+// (W x (np + nx + nq)). It holds all that the level needs: a serving kernel's
+// descriptors are written while it runs, and only the worker that claims a
+// root has an acquire behind it.
 __device__ __forceinline__ unsigned long long* idle_word(const KParams& kp, uint32_t i) {
     return kp.tctl + 16 * (1 + i);
 }
@@ -944,10 +946,10 @@ __device__ __forceinline__ size_t slot_need(uint32_t W, uint32_t npx, uint32_t n
 __device__ __forceinline__ bool slot_fits(const KParams& kp, uint32_t W, uint32_t npx, uint32_t nq) {
     return slot_need(W, npx, nq) <= kp.tslot_words && tree_wide_words(W, npx + nq, npx) <= kp.arena_words;
 }
-__device__ __forceinline__ void slot_head(u64* slot, uint32_t g, uint32_t W, uint32_t np,
+__device__ __forceinline__ void slot_head(u64* slot, const Walk& wk, uint32_t W, uint32_t np,
                                           uint32_t nx, uint32_t nq, u64 sr, u64 nr) {
     if (lane() == 0) {
-        st_rlx(slot, g);
+        st_rlx(slot, (u64)wk.g | ((u64)wk.r_is_u << 32));
         st_rlx(slot + 1, (u64)W | ((u64)np << 32));
         st_rlx(slot + 2, (u64)nx | ((u64)nq << 32));
         st_rlx(slot + 3, sr);
@@ -1023,7 +1025,7 @@ __device__ __forceinline__ bool donate_wide(const KParams& kp, const Wide& S, ui
             ix += __popcll(xw);
             iq += __popcll(qw);
         }
-        slot_head(slot, wk.g, W, np, nx, nq, F[1], F[2]);
+        slot_head(slot, wk, W, np, nx, nq, F[1], F[2]);
         hand_over(kp, to);
         for (uint32_t b = lane(); b < Wc; b += 64) {
             const u64 pw = P[b];
@@ -1080,7 +1082,7 @@ __device__ __forceinline__ bool donate_tile(const KParams& kp, const TileSrc& sr
             for (uint32_t q = lane(); q < src.nq; q += 64)
                 st_rlx(r + q0 + q, src.row(list[kTileP + q], i) & L);
         }
-        slot_head(slot, wk.g, W, np, nx, nq, uni64(F[64 * (C + 3)]), (uint32_t)uni64(F[64 * (C + 4)]));
+        slot_head(slot, wk, W, np, nx, nq, uni64(F[64 * (C + 3)]), (uint32_t)uni64(F[64 * (C + 4)]));
         hand_over(kp, to);
         if (lane() == 0) {
             F[64 * C] = A;
@@ -1718,7 +1720,9 @@ __global__ __launch_bounds__(64, 2) void mbe_tree(KParams kp) {
                 idle = false;
                 if (SEC) sec.mark(kSecWait);
                 u64* slot = slot_of(kp, wid);
-                wk.g = (uint32_t)uni64(ld_rlx(slot));
+                const u64 s0 = uni64(ld_rlx(slot));
+                wk.g = (uint32_t)s0;
+                wk.r_is_u = uni1((s0 >> 32) != 0);
                 start = stop ? kTreeOverflow : load_tree_slot(kp, slot, arena, lds_mem, S, src, M, list);
                 failed = start < 0;
                 dropped += failed && !stop;
@@ -1730,9 +1734,9 @@ __global__ __launch_bounds__(64, 2) void mbe_tree(KParams kp) {
         }
         if (got) {
             backoff = 1;
-            const DevGraph G = kp.graphs[wk.g];
-            wk.r_is_u = uni1(G.r_is_u);
             if (x != 0xFFFFFFFFu) {
+                const DevGraph G = kp.graphs[wk.g];
+                wk.r_is_u = uni1(G.r_is_u);
                 if (kp.serve) task = uni64(G.task_base) + x;
                 else x = (uint32_t)(task - uni64(G.task_base));
                 if (SEC) sec.mark(kSecOther);

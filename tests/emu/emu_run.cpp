@@ -12,7 +12,8 @@
 //           publishes each request's packed CSR to the kernel's mailbox, then
 //           closes it; prints "req <i> count <n> hash <0x...> err <e>" per
 //           request; a request is b<seed> (a batch graph) or
-//           c<n_u>,<n_v>,<m>,<gamma_u>,<gamma_v>,<max_deg>,<seed>)
+//           c<n_u>,<n_v>,<m>,<gamma_u>,<gamma_v>,<max_deg>,<seed> or
+//           e<n_u>,<n_v>,<p>,<n_planted>,<lo>,<hi>,<top_frac>,<seed>)
 // Options: -v variant(0..3) -w workers -l lds_words -a arena_words -s slots
 //          -c list_cutoff -r compact_ratio -i donate_interval -t twins(0|2)
 //          -b root_begin -e root_end -k root_stride -S side(-1|0|1)
@@ -20,6 +21,9 @@
 //          -x split_nodes (long tasks donate while the deque is short; 0 = never)
 //          -L large_edges (serve: requests with at least this many edges take
 //             the large claim lane) -T table_cap (serve) -u publish gap (us)
+//          -Z ms (serve): once all roots of a graph are claimed, and ms later,
+//             turn its descriptor's r_is_u round, as a cache line of before the
+//             graph was appended would hold something else
 //          -G seed of the garbage that fills uncleared device buffers
 //          -D us: a late atomic (wave_emu.h) lingers up to us after the next
 //             one, by a random sequence of seed -G
@@ -47,7 +51,7 @@ using namespace mbe;
 struct Opt {
     int variant = 0, side = -1;
     uint32_t sparse = 0, split = 0;
-    uint32_t large_edges = 1u << 18, table_cap = 64, gap_us = 0;
+    uint32_t large_edges = 1u << 18, table_cap = 64, gap_us = 0, stale_ms = 0;
     uint32_t workers = 8, lds_words = 3072, slots = 64, cutoff = 0, ratio = 2, interval = 64,
              twins = 1, rb = 0, re = 0, rs = 1;
     uint64_t arena_words = 1u << 18;
@@ -166,6 +170,16 @@ static int serve_main(const Opt& o, int n, char** specs) {
                 return 2;
             }
             g = gen_chung_lu(nu, nv, m, gu, gv, md, seed);
+        } else if (s[0] == 'e') {
+            unsigned nu, nv, np, lo, hi;
+            double p, top;
+            unsigned long long seed;
+            if (sscanf(s.c_str() + 1, "%u,%u,%lf,%u,%u,%u,%lf,%llu", &nu, &nv, &p, &np, &lo, &hi,
+                       &top, &seed) != 8) {
+                fprintf(stderr, "bad request %s\n", s.c_str());
+                return 2;
+            }
+            g = gen_er_planted(nu, nv, p, np, lo, hi, top, seed);
         } else {
             fprintf(stderr, "bad request %s\n", s.c_str());
             return 2;
@@ -282,8 +296,21 @@ static int serve_main(const Opt& o, int n, char** specs) {
             std::this_thread::sleep_for(std::chrono::microseconds(50));
         __atomic_store_n(flags + 2, 1ull, __ATOMIC_RELEASE);
     });
+    std::atomic<bool> over{false};
+    std::thread stale([&] {
+        for (int r = 0; o.stale_ms && r < n; r++) {
+            while (!over.load() &&
+                   (__atomic_load_n(flags + 1, __ATOMIC_ACQUIRE) <= (unsigned long long)r ||
+                    __atomic_load_n(&kp.root_cursor[r], __ATOMIC_ACQUIRE) < ps[r].n_roots))
+                std::this_thread::sleep_for(std::chrono::milliseconds(1));
+            std::this_thread::sleep_for(std::chrono::milliseconds(o.stale_ms));
+            if (!over.load()) gtable[r].r_is_u ^= 1;
+        }
+    });
     run_pass(kp, workers);
+    over.store(true);
     host.join();
+    stale.join();
     int bad = 0;
     for (int r = 0; r < n; r++) {
         const unsigned long long* d = done + 4 * r;
@@ -322,6 +349,7 @@ int main(int argc, char** argv) {
             case 'T': o.table_cap = (uint32_t)v; break;
             case 'u': o.gap_us = (uint32_t)v; break;
             case 'G': g_fill_seed = emu::g_linger_seed = (uint64_t)v; break;
+            case 'Z': o.stale_ms = (uint32_t)v; break;
             case 'D': emu::g_linger_us = (uint32_t)v; break;
             case 'P': g_progress_s = (uint32_t)v; break;
             default: fprintf(stderr, "unknown option -%c\n", f); return 2;

@@ -92,3 +92,18 @@ def test_late_count_keeps_idle_workers(workers, emu):
                                            "-G", seed, "er", *PLANTED)
         assert (count, h) == (ref.count, ref.hash), seed
         assert donated == stolen > 0
+
+
+def test_handed_level_needs_no_descriptor():
+    """A serving kernel's descriptors are written while it runs, and a worker
+    that takes a handed-over level may hold an older copy of their cache lines:
+    with the descriptor changed once all roots are claimed, the hash stays."""
+    spec = (300, 18, 0.6, 0, 0, 0, 0, 1)
+    ref = O.solve(*M.Graph.er_planted(*spec).csr())
+    subprocess.run(["make", "-C", EMU_DIR], check=True, capture_output=True)
+    out = subprocess.run([os.path.join(EMU_DIR, "emu_run"), "-w", "8", "-i", "1", "-S", "1", "-Z", "1000",
+                          "serve", "e" + ",".join(map(str, spec))],
+                         capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stderr + out.stdout
+    assert f"count {ref.count} hash {ref.hash:#018x} err 0 done 1" in out.stdout
+    assert int(re.search(r"stolen (\d+)", out.stdout).group(1)) > 0
