@@ -112,19 +112,23 @@ struct Walk {
     bool r_is_u, stop;
 };
 
-// Steps between two events: the donation interval, shorter under a node
-// budget so that a small budget is seen in time.
+constexpr uint32_t kWatchSteps = 1024;  // some 100 us
+__device__ __forceinline__ uint32_t give_interval(const KParams& kp) {
+    return kp.donate_interval ? kp.donate_interval : 64;
+}
+// Steps between two events: the donation interval, but under a watchdog no
+// more than kWatchSteps, and less under a node budget so that a small budget
+// is seen in time.
 __device__ __forceinline__ uint32_t event_interval(const KParams& kp) {
-    const uint32_t n = kp.donate_interval ? kp.donate_interval : 64;
-    return kp.node_budget ? min(n, 16u) : n;
+    return min(give_interval(kp), kp.node_budget ? 16u : kp.abort ? kWatchSteps : ~0u);
 }
 
 // Watchdog: charge the steps since the last look, look at the abort flag.
 // Every worker looks at the same line, so without a node budget it does every
-// 1,024 steps (some 100 us) and not at every event: with 2,048 workers that
-// took a batch of 64 graphs under a time limit from 16 ms to 23.
+// kWatchSteps and not at every event: with 2,048 workers that took a batch of
+// 64 graphs under a time limit from 16 ms to 23.
 __device__ __forceinline__ void watch(const KParams& kp, Walk& k) {
-    if (!kp.abort || (!kp.node_budget && k.steps - k.charged < 1024)) return;
+    if (!kp.abort || (!kp.node_budget && k.steps - k.charged < kWatchSteps)) return;
     if (charge_nodes(kp, k.steps - k.charged)) k.stop = true;
     k.charged = k.steps;
 }
@@ -433,7 +437,12 @@ constexpr uint32_t kNoX = 64;  // x of a frame without one in progress
 __device__ __forceinline__ bool event(const KParams& kp, Walk& k) {
     k.next_event = k.steps + event_interval(kp);
     watch(kp, k);
-    k.give = kp.variant != kNoWS ? uni32(may_give(kp, k)) : 0;
+    // the watchdog's events may be closer than the donation interval: then
+    // donation takes one in so many, at random
+    const uint32_t every = kp.abort ? give_interval(kp) / event_interval(kp) : 1;
+    const uint32_t h = (blockIdx.x * 0x85EBCA6Bu + (uint32_t)k.steps * 0x9E3779B1u) >> 4;
+    const uint32_t turn = every > 1 ? h % every : 0;
+    k.give = kp.variant != kNoWS && !turn ? uni32(may_give(kp, k)) : 0;
     return k.stop || k.give;
 }
 

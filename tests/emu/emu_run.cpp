@@ -27,6 +27,8 @@
 //          -G seed of the garbage that fills uncleared device buffers
 //          -D us: a late atomic (wave_emu.h) lingers up to us after the next
 //             one, by a random sequence of seed -G
+//          -A ms: raise the abort flag ms after a pass starts (a time limit)
+//          -n nodes: node budget (prints "aborted" when it is reached)
 //          -P s: print the workers' progress every s seconds (stderr)
 #include "wave_emu.h"
 #include "../../cumbe_amd/csrc/mbe_kernel.hip"
@@ -54,7 +56,7 @@ struct Opt {
     uint32_t large_edges = 1u << 18, table_cap = 64, gap_us = 0, stale_ms = 0;
     uint32_t workers = 8, lds_words = 3072, slots = 64, cutoff = 0, ratio = 2, interval = 64,
              twins = 1, rb = 0, re = 0, rs = 1;
-    uint64_t arena_words = 1u << 18;
+    uint64_t arena_words = 1u << 18, budget = 0;
 };
 
 template <int V>
@@ -69,6 +71,8 @@ constexpr size_t kLdsEmuWords = sizeof(lds_mem) / sizeof(u64);
 // With -P s: print the workers' finished roots and nodes (their progress
 // slots) every s seconds while a pass runs, to tell a slow run from a stuck one.
 static uint32_t g_progress_s = 0;
+// With -A ms: the host's part of a time limit.
+static uint32_t g_abort_ms = 0;
 
 static void run_pass(KParams& kp, uint32_t workers) {
     void (*fn)(void*) = kp.variant == 1 ? wave_fn<1> : kp.variant == 2 ? wave_fn<2>
@@ -92,6 +96,15 @@ static void run_pass(KParams& kp, uint32_t workers) {
                 fprintf(stderr, "progress %.0f s: roots %llu nodes %llu\n", s, r, nd);
             }
         });
+    std::thread limit;
+    if (g_abort_ms)
+        limit = std::thread([&] {
+            const auto t0 = std::chrono::steady_clock::now();
+            while (!pass_done.load() &&
+                   std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(g_abort_ms))
+                std::this_thread::sleep_for(std::chrono::milliseconds(1));
+            if (!pass_done.load()) __atomic_store_n(kp.abort, 1ull, __ATOMIC_SEQ_CST);
+        });
     if (kp.lds_words > kLdsEmuWords) {
         fprintf(stderr, "emu_run: lds_words %u beyond the emulated %zu\n", kp.lds_words,
                 kLdsEmuWords);
@@ -112,6 +125,7 @@ static void run_pass(KParams& kp, uint32_t workers) {
     for (auto& t : th) t.join();
     pass_done.store(true);
     if (mon.joinable()) mon.join();
+    if (limit.joinable()) limit.join();
 }
 
 static void* zalloc(size_t bytes) {
@@ -242,6 +256,7 @@ static int serve_main(const Opt& o, int n, char** specs) {
     kp.split_nodes = o.split;
     kp.abort = flags + 3;
     kp.node_count = kp.stats + kStatNodeBudget;
+    kp.node_budget = o.budget;
     kp.overflow_list = (uint64_t*)dalloc(ovf_cap * 8);
     kp.overflow_cap = ovf_cap;
     kp.slots = (uint64_t*)dalloc((size_t)o.slots * slot_words * 8);
@@ -349,6 +364,8 @@ int main(int argc, char** argv) {
             case 'T': o.table_cap = (uint32_t)v; break;
             case 'u': o.gap_us = (uint32_t)v; break;
             case 'G': g_fill_seed = emu::g_linger_seed = (uint64_t)v; break;
+            case 'A': g_abort_ms = (uint32_t)v; break;
+            case 'n': o.budget = (uint64_t)v; break;
             case 'Z': o.stale_ms = (uint32_t)v; break;
             case 'D': emu::g_linger_us = (uint32_t)v; break;
             case 'P': g_progress_s = (uint32_t)v; break;
@@ -437,6 +454,7 @@ int main(int argc, char** argv) {
         kp.split_nodes = o.split;
         kp.abort = &abort_flag;
         kp.node_count = kp.stats + kStatNodeBudget;
+        kp.node_budget = o.budget;
         kp.overflow_list = ovf;
         kp.overflow_cap = tasks.size();
         kp.slots = slots;
@@ -450,7 +468,7 @@ int main(int argc, char** argv) {
         free(kp.tctl);
         free(kp.tslots);
         launches++;
-        const uint64_t novf = ctl[1];
+        const uint64_t novf = abort_flag ? 0 : ctl[1];
         std::vector<uint64_t> next(ovf, ovf + novf);
         free(arena);
         free(mark);
@@ -464,8 +482,8 @@ int main(int argc, char** argv) {
     }
     const unsigned long long* st = ctl + 2;
     const unsigned long long* res = ctl + 2 + kStatCount + kSecCount;
-    printf("count %llu hash 0x%016llx nodes %llu donated %llu stolen %llu dropped %llu launches %u\n",
+    printf("count %llu hash 0x%016llx nodes %llu donated %llu stolen %llu dropped %llu launches %u%s\n",
            res[0], res[1], st[kStatNodes], st[kStatDonated], st[kStatStolen], st[kStatDropped],
-           launches);
+           launches, abort_flag ? " aborted" : "");
     return st[kStatDropped] ? 5 : 0;
 }

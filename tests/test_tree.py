@@ -10,6 +10,7 @@ windows before it and its Q those after it, up to d / s of each.
 import os
 import re
 import subprocess
+import time
 
 import pytest
 
@@ -107,3 +108,17 @@ def test_handed_level_needs_no_descriptor():
     assert out.returncode == 0, out.stderr + out.stdout
     assert f"count {ref.count} hash {ref.hash:#018x} err 0 done 1" in out.stdout
     assert int(re.search(r"stolen (\d+)", out.stdout).group(1)) > 0
+
+
+@pytest.mark.parametrize("opts", [(), ("-t", 0)], ids=["tree", "general"])
+def test_time_limit_without_donation(opts):
+    """The abort flag is seen within a task whatever the donation interval: a
+    root that takes many seconds here ends soon after the limit of 0.2 s."""
+    subprocess.run(["make", "-C", EMU_DIR], check=True, capture_output=True)
+    t0 = time.time()
+    out = subprocess.run([os.path.join(EMU_DIR, "emu_run"), "-w", "2", "-b", "16", "-e", "17", "-i",
+                          "4000000000", "-A", "200", *map(str, opts), "er", *map(str, PLANTED)],
+                         capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0 and out.stdout.endswith("aborted\n"), out.stderr + out.stdout
+    assert time.time() - t0 < 15
+    assert int(re.search(r"count (\d+)", out.stdout).group(1)) < 1 << 16
