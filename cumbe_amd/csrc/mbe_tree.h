@@ -105,7 +105,8 @@ struct Walk {
     u64 nodes, donated, words;
     u64 steps;       // vertices taken (the watchdog's and the donation's clock)
     u64 next_event;  // steps at which donation and the watchdog are looked at
-    u64 charged;     // steps charged against the node budget
+    u64 charged;     // nodes charged against the node budget; without one, the
+                     // steps at the last look at the abort flag
     u64 idle;        // lane i: idle workers of the i-th map word looked at
     uint32_t look;   // the first map word looked at
     uint32_t g, give;  // give: levels to give away at this event
@@ -123,14 +124,17 @@ __device__ __forceinline__ uint32_t event_interval(const KParams& kp) {
     return min(give_interval(kp), kp.node_budget ? 16u : kp.abort ? kWatchSteps : ~0u);
 }
 
-// Watchdog: charge the steps since the last look, look at the abort flag.
-// Every worker looks at the same line, so without a node budget it does every
-// kWatchSteps and not at every event: with 2,048 workers that took a batch of
-// 64 graphs under a time limit from 16 ms to 23.
+// Watchdog: charge the nodes since the last look (as mbe_result.nodes counts
+// them; steps are no measure, a wide step counts for many), look at the abort
+// flag. Every worker looks at the same line, so without a node budget it does
+// every kWatchSteps and not at every event: with 2,048 workers that took a
+// batch of 64 graphs under a time limit from 16 ms to 23.
 __device__ __forceinline__ void watch(const KParams& kp, Walk& k) {
-    if (!kp.abort || (!kp.node_budget && k.steps - k.charged < kWatchSteps)) return;
-    if (charge_nodes(kp, k.steps - k.charged)) k.stop = true;
-    k.charged = k.steps;
+    if (!kp.abort) return;
+    const u64 now = kp.node_budget ? k.nodes : k.steps;
+    if (!kp.node_budget && now - k.charged < kWatchSteps) return;
+    if (charge_nodes(kp, now - k.charged)) k.stop = true;
+    k.charged = now;
 }
 
 // ------------------------------------------------------------ hand-over

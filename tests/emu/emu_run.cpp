@@ -27,6 +27,7 @@
 //          -G seed of the garbage that fills uncleared device buffers
 //          -D us: a late atomic (wave_emu.h) lingers up to us after the next
 //             one, by a random sequence of seed -G
+//          -g 1: the general engine for the first pass, too
 //          -A ms: raise the abort flag ms after a pass starts (a time limit)
 //          -n nodes: node budget (prints "aborted" when it is reached)
 //          -P s: print the workers' progress every s seconds (stderr)
@@ -57,6 +58,7 @@ struct Opt {
     uint32_t workers = 8, lds_words = 3072, slots = 64, cutoff = 0, ratio = 2, interval = 64,
              twins = 1, rb = 0, re = 0, rs = 1;
     uint64_t arena_words = 1u << 18, budget = 0;
+    bool general = false;
 };
 
 template <int V>
@@ -153,12 +155,19 @@ static void* dalloc(size_t bytes) {
     return p;
 }
 
+// Words that waves share: their atomics may be late (wave_emu.h).
+static void* shared(void* p, size_t words) {
+    emu::late_words(p, words);
+    return p;
+}
+
 // The tree engine's control block and slots (host engine: setup_pass).
 static void tree_setup(KParams& kp, uint32_t workers, bool on) {
     kp.tree = on;
     if (!on) return;
     kp.tworkers = workers;
-    kp.tctl = (unsigned long long*)zalloc((size_t)tree_ctl_words(workers) * 8);
+    const size_t n = tree_ctl_words(workers);
+    kp.tctl = (unsigned long long*)shared(zalloc(n * 8), n);
     kp.tslot_words = std::min<uint64_t>(std::max<uint64_t>(1024, kp.arena_words), 1u << 16);
     kp.tslots = (uint64_t*)dalloc(kp.tslot_words * workers * 8);
 }
@@ -222,13 +231,13 @@ static int serve_main(const Opt& o, int n, char** specs) {
     MailRec* mail = (MailRec*)zalloc(cap * sizeof(MailRec));
     unsigned long long* flags = (unsigned long long*)zalloc(8 * 8);  // pub, taken, close, abort
     unsigned long long* done = (unsigned long long*)zalloc((size_t)cap * 32);
-    unsigned long long* rem = (unsigned long long*)dalloc((size_t)cap * 32);
+    unsigned long long* rem = (unsigned long long*)shared(dalloc((size_t)cap * 32), 4 * (size_t)cap);
     DevGraph* gtable = (DevGraph*)dalloc(cap * sizeof(DevGraph));
     ServeCtl* sctl = (ServeCtl*)zalloc(sizeof(ServeCtl));
     const uint64_t mark_words = (max_nr + 255) / 256 * 4, cpos_len = max_nr + 1;
     const size_t ctl_words = 2 + kStatCount + kSecCount + 2 * (size_t)cap;
-    unsigned long long* ctl = (unsigned long long*)zalloc(ctl_words * 8);
-    unsigned long long* dq = (unsigned long long*)zalloc((4 + o.slots) * 8);
+    unsigned long long* ctl = (unsigned long long*)shared(zalloc(ctl_words * 8), ctl_words);
+    unsigned long long* dq = (unsigned long long*)shared(zalloc((4 + o.slots) * 8), 4 + o.slots);
     for (uint32_t s = 0; s < o.slots; s++) dq[4 + s] = s;
     const uint32_t workers = o.workers;
     const uint64_t arena_words = o.arena_words;
@@ -277,7 +286,7 @@ static int serve_main(const Opt& o, int n, char** specs) {
     kp.data = data;
     kp.close = flags + 2;
     kp.done = done;
-    tree_setup(kp, workers, o.twins);
+    tree_setup(kp, workers, o.twins && !o.general);
     std::thread host([&] {
         for (int r = 0; r < n; r++) {
             if (o.gap_us) std::this_thread::sleep_for(std::chrono::microseconds(o.gap_us));
@@ -364,9 +373,11 @@ int main(int argc, char** argv) {
             case 'T': o.table_cap = (uint32_t)v; break;
             case 'u': o.gap_us = (uint32_t)v; break;
             case 'G': g_fill_seed = emu::g_linger_seed = (uint64_t)v; break;
+            case 'g': o.general = v != 0; break;
             case 'A': g_abort_ms = (uint32_t)v; break;
             case 'n': o.budget = (uint64_t)v; break;
             case 'Z': o.stale_ms = (uint32_t)v; break;
+            
             case 'D': emu::g_linger_us = (uint32_t)v; break;
             case 'P': g_progress_s = (uint32_t)v; break;
             default: fprintf(stderr, "unknown option -%c\n", f); return 2;
@@ -411,8 +422,8 @@ int main(int argc, char** argv) {
 
     const uint64_t mark_words = ((uint64_t)p.nR + 255) / 256 * 4 + 4, cpos_len = (uint64_t)p.nR + 1;
     const size_t ctl_words = 2 + kStatCount + kSecCount + 2;
-    unsigned long long* ctl = (unsigned long long*)zalloc(ctl_words * 8);
-    unsigned long long* dq = (unsigned long long*)zalloc((4 + o.slots) * 8);
+    unsigned long long* ctl = (unsigned long long*)shared(zalloc(ctl_words * 8), ctl_words);
+    unsigned long long* dq = (unsigned long long*)shared(zalloc((4 + o.slots) * 8), 4 + o.slots);
     unsigned long long abort_flag = 0;
     uint64_t arena_words = o.arena_words;
     uint32_t workers = o.workers;
@@ -463,7 +474,7 @@ int main(int argc, char** argv) {
         kp.donate_interval = o.interval;
         kp.dq = dq;
         kp.progress = progress;
-        tree_setup(kp, workers, o.twins && !launches);
+        tree_setup(kp, workers, o.twins && !o.general && !launches);
         run_pass(kp, workers);
         free(kp.tctl);
         free(kp.tslots);
@@ -485,5 +496,6 @@ int main(int argc, char** argv) {
     printf("count %llu hash 0x%016llx nodes %llu donated %llu stolen %llu dropped %llu launches %u%s\n",
            res[0], res[1], st[kStatNodes], st[kStatDonated], st[kStatStolen], st[kStatDropped],
            launches, abort_flag ? " aborted" : "");
+    if (o.budget) printf("charged %llu\n", st[kStatNodeBudget]);
     return st[kStatDropped] ? 5 : 0;
 }

@@ -13,7 +13,8 @@
 // a thread_local array per wave.
 //
 // Nothing but a wait orders an atomic whose result is not used with the wave's
-// next one on another address, so it is performed late here: when the wave
+// next one on another address. On the words that waves share (late_words; a
+// wave's own memory is read back with plain loads) it is performed late: when the wave
 // waits (s_waitcnt, a fence, a release store), sleeps or touches the address
 // again, or after the next atomic that does return. There the wave first
 // lingers, up to g_linger_us at random, so that others see the later one alone.
@@ -76,7 +77,13 @@ struct Late {
     void (*perform)(void*, uint64_t);
     uint64_t v;
 };
-constexpr size_t kMaxLate = 64;
+struct Span {
+    const char *begin, *end;
+};
+inline std::vector<Span> g_shared;  // set before the waves start
+inline void late_words(const void* p, size_t n) {
+    g_shared.push_back({(const char*)p, (const char*)p + n * 8});
+}
 inline thread_local std::vector<Late> g_late;
 inline thread_local uint64_t g_rand = 0;
 inline uint32_t g_linger_us = 0;
@@ -127,8 +134,13 @@ struct Atomic {
     }
     ~Atomic() {
         if (read) return;
+        bool shared = false;
+        for (const Span& r : g_shared) shared |= (char*)p >= r.begin && (char*)p < r.end;
+        if (!shared) {
+            Op::perform(p, v);
+            return;
+        }
         perform_late(p);
-        if (g_late.size() == kMaxLate) perform_late();
         g_late.push_back({p, [](void* q, uint64_t w) { Op::perform((T*)q, (T)w); }, (uint64_t)v});
     }
 };

@@ -122,3 +122,19 @@ def test_time_limit_without_donation(opts):
     assert out.returncode == 0 and out.stdout.endswith("aborted\n"), out.stderr + out.stdout
     assert time.time() - t0 < 15
     assert int(re.search(r"count (\d+)", out.stdout).group(1)) < 1 << 16
+
+
+def test_node_budget_counts_nodes(emu, tmp_path):
+    """The node budget is in nodes of the tree as they are reported, on wide
+    levels too (some 300 candidates a root here): a budget that covers them
+    does not stop the solve, a quarter of it does."""
+    import random
+    rng = random.Random(1)
+    g = csr_from_edges(600, 800, [(i, j) for i in range(600) for j in rng.sample(range(800), 8)])
+    ref = O.solve(*g)
+    path = str(tmp_path / "sparse.bi")
+    M.Graph.from_csr(*g).write_bi(path)
+    nodes = emu("-w", 4, "-S", 0, "bi", path)[2]
+    count, h, *_ = emu("-w", 4, "-S", 0, "-n", nodes + 1, "bi", path)
+    assert (count, h) == (ref.count, ref.hash)
+    assert emu("-w", 4, "-S", 0, "-n", nodes // 4, "bi", path)[0] < ref.count
