@@ -174,6 +174,7 @@ __device__ __forceinline__ bool charge_nodes(const KParams& kp, u64 n) {
         total = atomicAdd(kp.node_count, n) + n;
         if (total >= kp.node_budget) {
             st_rlx(kp.stats + kStatAbortSeen, 1ull);
+            if (kp.serve) st_rlx(&kp.serve->abort_seen, 1ull);
             __hip_atomic_store(kp.abort, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }

@@ -95,16 +95,26 @@ def test_late_count_keeps_idle_workers(workers, emu):
         assert donated == stolen > 0
 
 
+def serve_emu(*args):
+    subprocess.run(["make", "-C", EMU_DIR], check=True, capture_output=True)
+    return subprocess.run([os.path.join(EMU_DIR, "emu_run"), *map(str, args)], capture_output=True,
+                          text=True, timeout=300)
+
+
+def test_served_node_budget_stops_busy_workers():
+    """A serving kernel's node budget stops workers that never idle: the only
+    worker, with 14 roots of a request before it, reports a part of it."""
+    out = serve_emu("-w", 1, "-S", 1, "-n", 500, "serve", "e120,14,0.7,0,0,0,0,1")
+    assert int(re.search(r"nodes (\d+)", out.stdout).group(1)) < 2000, out.stdout + out.stderr
+
+
 def test_handed_level_needs_no_descriptor():
     """A serving kernel's descriptors are written while it runs, and a worker
     that takes a handed-over level may hold an older copy of their cache lines:
     with the descriptor changed once all roots are claimed, the hash stays."""
     spec = (300, 18, 0.6, 0, 0, 0, 0, 1)
     ref = O.solve(*M.Graph.er_planted(*spec).csr())
-    subprocess.run(["make", "-C", EMU_DIR], check=True, capture_output=True)
-    out = subprocess.run([os.path.join(EMU_DIR, "emu_run"), "-w", "8", "-i", "1", "-S", "1", "-Z", "1000",
-                          "serve", "e" + ",".join(map(str, spec))],
-                         capture_output=True, text=True, timeout=300)
+    out = serve_emu("-w", 8, "-i", 1, "-S", 1, "-Z", 1000, "serve", "e" + ",".join(map(str, spec)))
     assert out.returncode == 0, out.stderr + out.stdout
     assert f"count {ref.count} hash {ref.hash:#018x} err 0 done 1" in out.stdout
     assert int(re.search(r"stolen (\d+)", out.stdout).group(1)) > 0
