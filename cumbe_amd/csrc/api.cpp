@@ -299,8 +299,9 @@ struct Emit {
     uint64_t cap = 0;
 };
 
-// Run every root task of the uploaded graphs; roots whose local problem does
-// not fit a worker arena are retried with fewer workers and larger arenas.
+// Run every root task of the uploaded graphs; roots that the tree engine
+// leaves run on the general engine, and those whose local problem does not fit
+// a worker arena with fewer workers and larger arenas.
 mbe_status run_tasks(Engine& E, Bufs& B, const Meta& m, int variant, const Tune& tu,
                      std::vector<uint64_t>& res, mbe_result& out, const Pass0* pre = nullptr,
                      const Emit* em = nullptr) {
@@ -311,6 +312,7 @@ mbe_status run_tasks(Engine& E, Bufs& B, const Meta& m, int variant, const Tune&
     uint64_t n_tasks = m.total_tasks;
     uint64_t arena_words = tu.arena_words;
     uint32_t workers = tu.workers;
+    const bool tree_first = !(tu.flags & MBE_FLAG_REFERENCE_TREE);
     std::vector<uint64_t> task_list;  // empty = range mode
     if (m.ng == 1 && (tu.root_begin || tu.root_end || tu.root_stride > 1)) {
         const uint64_t end = tu.root_end ? std::min<uint64_t>(tu.root_end, m.total_tasks) : m.total_tasks;
@@ -324,7 +326,8 @@ mbe_status run_tasks(Engine& E, Bufs& B, const Meta& m, int variant, const Tune&
     __atomic_store_n(E.abort_flag, 0ull, __ATOMIC_SEQ_CST);
     mbe::KParams kp{};
     for (int pass = 0; n_tasks > 0; pass++) {
-        if (pass > 6) return fail(MBE_ENOMEM, "root subproblem does not fit any arena");
+        if (pass >= mbe::kMaxPasses + (tree_first ? 1 : 0))
+            return fail(MBE_ENOMEM, "root subproblem does not fit any arena");
         uint32_t nw = workers;  // all start: those without a root task steal
         if (pass == 0 && pre) {
             kp = pre->kp;
@@ -362,7 +365,7 @@ mbe_status run_tasks(Engine& E, Bufs& B, const Meta& m, int variant, const Tune&
         task_list.resize(novf);
         HIPC(hipMemcpy(task_list.data(), kp.overflow_list, novf * 8, hipMemcpyDeviceToHost));
         n_tasks = novf;
-        arena_words *= 16;
+        arena_words = mbe::next_arena_words(arena_words, pass == 0 && tree_first);
         workers = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(workers, budget_words / arena_words));
     }
     if (!launches) {  // no root task at all: every graph has count 0
@@ -818,10 +821,11 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
     uint32_t launches = 0, used_workers = 0;
     mbe::KParams kp{};
     for (int pass = 0; n_tasks > 0; pass++) {
-        if (pass > 6) return fail(MBE_ERANGE, "root subproblem does not fit an arena of the scratch");
+        const bool tree = pass == 0 && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
+        if (pass >= mbe::kMaxPasses + (kp.twins ? 1 : 0))
+            return fail(MBE_ERANGE, "root subproblem does not fit an arena of the scratch");
         const uint64_t slot_words = std::min<uint64_t>(std::max<uint64_t>(4096, arena_words), 1u << 19);
         const uint64_t w_slots = up4(kNoAllocSlots * slot_words);
-        const bool tree = pass == 0 && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
         // the tree engine's hand-over: a slot and, of the control block, a
         // flag line and a share of the idle map per worker
         const uint64_t tslot_words = std::min(tree_slot_words(arena_words), kNoAllocTreeSlotWords);
@@ -905,7 +909,7 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
         HIPC(hipMemcpy(&novf, kp.overflow_count, 8, hipMemcpyDeviceToHost));
         if (__atomic_load_n(E.abort_flag, __ATOMIC_SEQ_CST) || !novf) break;
         n_tasks = novf;
-        arena_words *= 16;
+        arena_words = mbe::next_arena_words(arena_words, tree);
         workers = nw;
     }
     unsigned long long st[mbe::kStatCount], sc[mbe::kSecCount], rr[2];

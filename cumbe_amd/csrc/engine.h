@@ -87,6 +87,15 @@ constexpr uint64_t tree_root_words(uint64_t d, uint64_t nc) {
     return (nc + 1) / 2 + nc + 1 + tree_wide_words(W, nc, nc < d ? nc : d) + nc * W;
 }
 
+// Arena words of the pass over the roots that a pass left: the tree engine
+// leaves those that list mode suits, and some whose layout alone did not fit,
+// so the general engine first tries at the same size; what it leaves has
+// overflowed its arena.
+constexpr uint64_t next_arena_words(uint64_t arena_words, bool after_tree) {
+    return after_tree ? arena_words : arena_words * 16;
+}
+constexpr int kMaxPasses = 7;  // over growing arenas, besides the tree engine's
+
 // Deque slot header for donated subtrees (see mbe_kernel.hip).
 constexpr uint32_t kSlotHeaderWords = 8;
 

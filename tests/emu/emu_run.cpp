@@ -428,9 +428,10 @@ int main(int argc, char** argv) {
     uint64_t arena_words = o.arena_words;
     uint32_t workers = o.workers;
     unsigned launches = 0;
+    uint64_t last_arena = 0;  // of the last pass
     KParams kp{};
     while (!tasks.empty()) {
-        if (launches > 6) { fprintf(stderr, "root does not fit any arena\n"); return 4; }
+        if (launches > kMaxPasses) { fprintf(stderr, "root does not fit any arena\n"); return 4; }
         const uint64_t slot_words = std::min<uint64_t>(std::max<uint64_t>(4096, arena_words), 1u << 19);
         uint64_t* arena = (uint64_t*)dalloc(arena_words * workers * 8);
         uint64_t* mark = (uint64_t*)zalloc(mark_words * workers * 8);
@@ -479,6 +480,7 @@ int main(int argc, char** argv) {
         free(kp.tctl);
         free(kp.tslots);
         launches++;
+        last_arena = arena_words;
         const uint64_t novf = abort_flag ? 0 : ctl[1];
         std::vector<uint64_t> next(ovf, ovf + novf);
         free(arena);
@@ -488,14 +490,15 @@ int main(int argc, char** argv) {
         free(ovf);
         free(progress);
         tasks.swap(next);
-        arena_words *= 16;
-        workers = std::max<uint32_t>(1, std::min<uint32_t>(workers, 4));
+        arena_words = next_arena_words(arena_words, kp.tree);
+        if (!kp.tree) workers = std::max<uint32_t>(1, std::min<uint32_t>(workers, 4));
     }
     const unsigned long long* st = ctl + 2;
     const unsigned long long* res = ctl + 2 + kStatCount + kSecCount;
     printf("count %llu hash 0x%016llx nodes %llu donated %llu stolen %llu dropped %llu launches %u%s\n",
            res[0], res[1], st[kStatNodes], st[kStatDonated], st[kStatStolen], st[kStatDropped],
            launches, abort_flag ? " aborted" : "");
+    printf("arena %llu\n", (unsigned long long)last_arena);
     if (o.budget) printf("charged %llu\n", st[kStatNodeBudget]);
     return st[kStatDropped] ? 5 : 0;
 }

@@ -101,3 +101,9 @@ def wide_twins(seed=5, d=4200, n_l=6000, n_c=6):
     rows += sets
     edges = [(u, v) for u, r in enumerate(rows) for v in r]
     return csr_from_edges(len(rows), n_l, edges)
+
+
+def star_of_stars(n=1000):
+    """Column 0 is adjacent to n rows, and each row to one column of its own:
+    column 0's local problem is n x n bits of which n are set."""
+    return csr_from_edges(n, n + 1, [(i, j) for i in range(n) for j in (0, i + 1)])

@@ -15,7 +15,7 @@ import time
 import pytest
 
 import oracle_lib as O
-from graphs import csr_from_edges
+from graphs import csr_from_edges, star_of_stars
 
 M = pytest.importorskip("cumbe_amd")
 EMU_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "emu")
@@ -148,3 +148,15 @@ def test_node_budget_counts_nodes(emu, tmp_path):
     count, h, *_ = emu("-w", 4, "-S", 0, "-n", nodes + 1, "bi", path)
     assert (count, h) == (ref.count, ref.hash)
     assert emu("-w", 4, "-S", 0, "-n", nodes // 4, "bi", path)[0] < ref.count
+
+
+def test_list_mode_root_keeps_the_arena_size(tmp_path):
+    """A root that the tree engine leaves to list mode fits the arenas that
+    there are: its pass does not ask for larger ones."""
+    g = star_of_stars()
+    ref = O.solve(*g)
+    path = str(tmp_path / "star.bi")
+    M.Graph.from_csr(*g).write_bi(path)
+    out = serve_emu("-p", 8, "-a", 32768, "-S", 1, "bi", path).stdout
+    assert out.startswith(f"count {ref.count} hash {ref.hash:#018x}")
+    assert "launches 2" in out and "arena 32768" in out

@@ -16,6 +16,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 GOLD = os.path.join(ROOT, "tests", "golden")
 pytestmark = pytest.mark.gpu
 M = pytest.importorskip("cumbe_amd")
+import oracle_lib as O  # noqa: E402
+from graphs import star_of_stars  # noqa: E402
 
 
 class DevCopy:
@@ -39,7 +41,7 @@ def say(msg):
 
 
 def check(g, variant="cuMBE", tuning=None):
-    buf, info = g.pack()
+    buf, info = g.pack((tuning or {}).get("side", -1))
     dev = DevCopy(buf)
     try:
         r = M.solve_noalloc(dev.ptr.value, info, variant, tuning)
@@ -80,3 +82,26 @@ def test_noalloc_variants_subset_and_limits():
         assert e.value.status == -9
     finally:
         dev.close()
+
+
+def free_bytes():
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_list_mode_root_at_the_default_arena():
+    """A hub root that list mode suits is left to a second pass, at the same
+    arena size: it fits the scratch of the allocation-free solve, and a solve
+    takes no larger arenas for it (they would be 48 GiB)."""
+    M.init()
+    n_u, n_v, off, adj = star_of_stars()
+    g = M.Graph.from_csr(n_u, n_v, off, adj)
+    M.solve(M.Graph.chung_lu(400, 300, 2500, 2.1, 2.1, 0, 11))
+    before = free_bytes()
+    say("noalloc and solve with a list-mode root")
+    r = check(g, "cuMBE", {"side": 1})
+    ref = O.solve(n_u, n_v, off, adj)
+    assert (r.count, r.hash, r.launches) == (ref.count, ref.hash, 2)
+    assert before - free_bytes() < 8 << 30
