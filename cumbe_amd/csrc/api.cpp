@@ -186,30 +186,42 @@ hipError_t wait_with_progress(Engine& E, const Bufs& B, uint32_t nw, uint64_t n_
 
 
 
+// The general engine's ring: a slot holds a compacted level of any problem
+// that fits an arena, up to 4 MiB.
+uint64_t ring_slot_words(uint64_t arena_words) {
+    return std::min<uint64_t>(std::max<uint64_t>(4096, arena_words), 1u << 19);
+}
+
+PassSizes pass_sizes(const Meta& m, const Tune& tu, bool tree, uint64_t arena_words,
+                     uint32_t workers) {
+    PassSizes n;
+    n.need(&Bufs::ctl, m.ctl_words() * 8);
+    n.need(&Bufs::ovf, m.ovf_cap() * 8 * 2);
+    n.need(&Bufs::arena, arena_words * workers * 8);
+    n.need(&Bufs::mark, m.mark_words() * workers * 8);
+    n.need(&Bufs::cpos, m.cpos_len() * workers * 4);
+    if (tree) {  // hand-over: a slot per worker
+        n.need(&Bufs::tctl, (size_t)mbe::tree_ctl_words(workers) * 8);
+        n.need(&Bufs::tslots, tree_slot_words(arena_words) * workers * 8);
+    } else {
+        n.need(&Bufs::slots, (size_t)kSlots * ring_slot_words(arena_words) * 8);
+        n.need(&Bufs::dq, (4 + (size_t)kSlots) * 8);
+    }
+    if (tu.flags & MBE_FLAG_VARIANCE) n.need(&Bufs::busy, (size_t)workers * 8);
+    n.workers = workers;
+    return n;
+}
+
 // Size the buffers of one pass and fill its kernel parameters. The task list
 // (explicit global task ids, or none for all tasks) is copied to the device.
 mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_host, const Meta& m,
                       const Tune& tu, int variant, bool first,
                       const std::vector<uint64_t>& task_list, uint64_t n_tasks,
                       uint64_t arena_words, uint32_t workers, mbe::KParams& kp) {
-    HIPC(B.ctl.ensure(m.ctl_words() * 8));
-    const uint64_t ovf_cap = std::max<uint64_t>(m.total_tasks, 1);
-    HIPC(B.ovf.ensure(ovf_cap * 8 * 2));
-    HIPC(B.arena.ensure(arena_words * workers * 8));
-    HIPC(B.mark.ensure(m.mark_words() * workers * 8));
-    HIPC(B.cpos.ensure(m.cpos_len() * workers * 4));
-    // the general engine's ring: a slot holds a compacted level of any problem
-    // that fits an arena, up to 4 MiB per slot; the tree engine's hand-over: a
-    // slot per worker
     const bool tree = first && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
-    const uint64_t slot_words = std::min<uint64_t>(std::max<uint64_t>(4096, arena_words), 1u << 19);
-    if (tree) {
-        HIPC(B.tctl.ensure((size_t)mbe::tree_ctl_words(workers) * 8));
-        HIPC(B.tslots.ensure(tree_slot_words(arena_words) * workers * 8));
-    } else {
-        HIPC(B.slots.ensure((size_t)kSlots * slot_words * 8));
-        HIPC(B.dq.ensure((4 + (size_t)kSlots) * 8));
-    }
+    const uint64_t ovf_cap = m.ovf_cap();
+    for (const auto& n : pass_sizes(m, tu, tree, arena_words, workers).bufs)
+        HIPC((B.*n.first).ensure(n.second));
     HIPC(B.ensure_progress(workers));
     memset(B.progress, 0, 2 * (size_t)workers * 8);
     unsigned long long* ctl = B.ctl.as<unsigned long long>();
@@ -229,10 +241,7 @@ mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_hos
     kp.stats = ctl + 2;
     const bool variance = tu.flags & MBE_FLAG_VARIANCE;
     kp.sections = (tu.flags & MBE_FLAG_SECTIONS) || variance ? ctl + 2 + mbe::kStatCount : nullptr;
-    if (variance) {
-        HIPC(B.busy.ensure((size_t)workers * 8));
-        kp.worker_busy = B.busy.as<unsigned long long>();
-    }
+    if (variance) kp.worker_busy = B.busy.as<unsigned long long>();
     kp.results = ctl + 2 + mbe::kStatCount + mbe::kSecCount;
     kp.arena = B.arena.as<uint64_t>();
     kp.arena_words = arena_words;
@@ -260,7 +269,7 @@ mbe_status setup_pass(Bufs& B, hipStream_t stream, unsigned long long* abort_hos
     kp.donate_depth = tu.donate_depth;
     kp.donate_interval = tu.donate_interval;
     kp.slots = B.slots.as<uint64_t>();
-    kp.slot_words = slot_words;
+    kp.slot_words = ring_slot_words(arena_words);
     kp.n_slots = kSlots;
     kp.dq = B.dq.as<unsigned long long>();
     if (getenv("MBE_PROGRESS")) HIPC(hipHostGetDevicePointer((void**)&kp.progress, B.progress, 0));
@@ -824,7 +833,7 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
         const bool tree = pass == 0 && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
         if (pass >= mbe::kMaxPasses + (kp.twins ? 1 : 0))
             return fail(MBE_ERANGE, "root subproblem does not fit an arena of the scratch");
-        const uint64_t slot_words = std::min<uint64_t>(std::max<uint64_t>(4096, arena_words), 1u << 19);
+        const uint64_t slot_words = ring_slot_words(arena_words);
         const uint64_t w_slots = up4(kNoAllocSlots * slot_words);
         // the tree engine's hand-over: a slot and, of the control block, a
         // flag line and a share of the idle map per worker

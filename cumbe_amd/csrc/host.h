@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/mbe.h"
@@ -41,8 +42,8 @@ double now_ms();
         }                                                                                  \
     } while (0)
 
-// Free the device buffers that a destroyed server left for the next one (see
-// serve.cpp); whether there were any.
+// Free the buffers that a destroyed server left for the next one (see
+// serve.cpp), if no server is alive; whether there were any.
 bool give_back_kept();
 
 // Device buffer that grows on demand and is reused across solves.
@@ -122,6 +123,8 @@ struct Meta {
     // whole blocks of four words (see marked_below)
     uint64_t mark_words() const { return ((uint64_t)max_nr + 255) / 256 * 4; }
     uint64_t cpos_len() const { return (uint64_t)max_nr + 1; }
+    // roots that one pass may leave to the next
+    uint64_t ovf_cap() const { return std::max<uint64_t>(total_tasks, 1); }
     // control block: cursor, overflow count, stats, section ticks, results
     size_t ctl_words() const { return 2 + mbe::kStatCount + mbe::kSecCount + 2 * (size_t)ng; }
 };
@@ -152,6 +155,21 @@ mbe_status upload(Bufs& B, hipStream_t stream, const std::vector<const Prepared*
                   std::vector<DevGraph>& dg, uint64_t& total_tasks);
 
 Meta meta_of(const std::vector<const Prepared*>& ps, uint64_t total_tasks);
+
+// The buffers one pass needs, and their sizes in bytes.
+struct PassSizes {
+    std::vector<std::pair<DevBuf Bufs::*, size_t>> bufs;
+    uint32_t workers = 0;
+    void need(DevBuf Bufs::*b, size_t bytes) { bufs.emplace_back(b, bytes); }
+    // whether b holds them all, so that the pass allocates and frees nothing
+    bool fit(const Bufs& b) const {
+        for (const auto& n : bufs)
+            if ((b.*n.first).bytes < n.second) return false;
+        return b.progress_slots >= 2 * (size_t)workers;
+    }
+};
+PassSizes pass_sizes(const Meta& m, const Tune& tu, bool tree, uint64_t arena_words,
+                     uint32_t workers);
 
 // Size the buffers of one pass and fill its kernel parameters; abort_host is
 // the host-mapped watchdog flag the kernel polls. first: the first pass, which

@@ -30,8 +30,12 @@ using namespace mbe::host;
 // it gives it out again, so a program that creates a server per burst waited
 // 250 ms in every destroy once it had been through the card's memory (some 30
 // servers); the burst itself takes 14. One set is kept at most, and none above
-// 16 GiB; an allocation of this library that fails gives it back, unless a
-// server is alive: its kernel runs on, and a free would wait for that.
+// 16 GiB. A free waits for every kernel on the device, a live server's included,
+// and that one ends when its owner says so. So a server takes the set only when
+// it holds all that its launches need (it allocates and frees nothing then), and
+// the set is freed, under the lock that counts the servers, only while none is
+// alive: by a server that cannot use it, and by an allocation of this library
+// that fails.
 constexpr size_t kKeepBytes = (size_t)16 << 30;
 struct Kept {
     std::mutex m;
@@ -42,18 +46,25 @@ Kept& kept() {
     static Kept* k = new Kept();  // never destroyed: outlives HIP teardown
     return *k;
 }
-// The kept set, for a new server (servers: 1) or to be freed (0).
-Bufs take_kept(int servers) {
+// A server begins: the kept set, if that is enough for it.
+Bufs begin_server(const PassSizes& need) {
     std::lock_guard<std::mutex> lk(kept().m);
-    if (!servers && kept().servers) return Bufs{};
-    kept().servers += servers;
-    return std::exchange(kept().b, Bufs{});
+    Bufs b;
+    if (need.fit(kept().b))
+        std::swap(b, kept().b);
+    else if (kept().servers == 0)
+        kept().b.release();
+    kept().servers++;
+    return b;
 }
-// b's work has ended. Its buffers are kept, or else the ones kept before.
-void keep(Bufs& b) {
-    if (b.device_bytes() <= kKeepBytes) {
+// A server ends, its work done: its buffers b are kept, or else the ones kept
+// before; the others are freed.
+void end_server(Bufs& b, bool keep) {
+    {
         std::lock_guard<std::mutex> lk(kept().m);
-        if (b.device_bytes() > kept().b.device_bytes()) std::swap(b, kept().b);
+        kept().servers--;
+        if (keep && b.device_bytes() <= kKeepBytes && b.device_bytes() > kept().b.device_bytes())
+            std::swap(b, kept().b);
     }
     b.release();
 }
@@ -152,6 +163,7 @@ struct mbe_server {
     std::thread th;
     bool stop = false;
     bool failed = false;
+    bool counted = false;  // among the servers alive (see Kept)
     std::string fail_msg;
 
     // device side
@@ -170,16 +182,21 @@ struct mbe_server {
     Ring data_ring, stage_ring;
     std::deque<std::pair<uint64_t, uint64_t>> staged;  // (record seq, staging pos)
 
+    Meta meta() const {
+        Meta m;
+        m.ng = cfg.table_cap;
+        m.max_nr = cfg.max_nr;
+        m.total_tasks = 1u << 20;  // overflow-list capacity
+        return m;
+    }
+
     mbe_status launch_generation() {
         *mail_pub = 0;
         *mail_taken = 0;
         *close_flag = 0;
         *abort_flag = 0;
         memset(done, 0, (size_t)cfg.table_cap * 32);
-        Meta m;
-        m.ng = cfg.table_cap;
-        m.max_nr = cfg.max_nr;
-        m.total_tasks = 1u << 20;  // overflow-list capacity
+        const Meta m = meta();
         mbe_status s = setup_pass(b, stream, abort_flag, m, tu, 0, true, {}, 0,
                                   tu.arena_words, tu.workers, kp);
         if (s != MBE_OK) return s;
@@ -417,20 +434,18 @@ struct mbe_server {
 
 namespace mbe::host {
 bool give_back_kept() {
-    Bufs b = take_kept(0);
-    const bool any = b.device_bytes() != 0;
-    b.release();
-    return any;
+    std::lock_guard<std::mutex> lk(kept().m);
+    if (kept().servers || !kept().b.device_bytes()) return false;
+    kept().b.release();
+    return true;
 }
 }  // namespace mbe::host
 
 namespace {
 
 void free_server(mbe_server* S) {
-    if (S->stream && hipStreamSynchronize(S->stream) == hipSuccess && !S->failed)
-        keep(S->b);
-    else
-        S->b.release();
+    const bool done = S->stream && hipStreamSynchronize(S->stream) == hipSuccess && !S->failed;
+    if (S->counted) end_server(S->b, done);
     for (DevBuf* d : {&S->gtable, &S->rem, &S->sctl, &S->data}) {
         if (d->p) (void)hipFree(d->p);
         d->p = nullptr;
@@ -440,12 +455,9 @@ void free_server(mbe_server* S) {
         if (h) (void)hipHostFree(h);
     if (S->ev_end) (void)hipEventDestroy(S->ev_end);
     if (S->stream) (void)hipStreamDestroy(S->stream);
-    std::lock_guard<std::mutex> lk(kept().m);
-    kept().servers--;
 }
 
 mbe_status make_server(mbe_server* S) {
-    S->b = take_kept(1);
     HIPC(hipSetDevice(0));
     hipDeviceProp_t prop;
     HIPC(hipGetDeviceProperties(&prop, 0));
@@ -465,6 +477,9 @@ mbe_status make_server(mbe_server* S) {
         return fail(MBE_EINVAL, "root subsets are not served");
     mbe_status s = ensure_lds(S->tu.lds_words);
     if (s != MBE_OK) return s;
+    S->b = begin_server(pass_sizes(S->meta(), S->tu, !(S->tu.flags & MBE_FLAG_REFERENCE_TREE),
+                                   S->tu.arena_words, S->tu.workers));
+    S->counted = true;
     const uint64_t cap = S->cfg.table_cap;
     HIPC(hipStreamCreateWithFlags(&S->stream, hipStreamNonBlocking));
     HIPC(hipEventCreateWithFlags(&S->ev_end, hipEventDisableTiming));

@@ -1,6 +1,8 @@
-"""GPU test of the launch buffers that pass from a destroyed server to the next
+"""GPU tests of the launch buffers that pass from a destroyed server to the next
 one: servers that need more, less or the same as the one before, with a solve
-in between, all give the solve's result."""
+in between, all give the solve's result; and two servers at a time."""
+import threading
+
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -27,3 +29,30 @@ def test_server_after_server():
             burst(srv)
         r = M.solve(graphs[0])
         assert (r.count, r.hash) == want[0]
+
+
+def test_larger_server_beside_a_running_one():
+    """A small server has left its buffers; of two larger ones the second gets
+    its request first and keeps its kernel running. The first one's request
+    then completes: what it needs is allocated, and nothing is freed, which
+    would wait for the other's kernel."""
+    g = M.Graph.chung_lu(300, 150, 1500, 2.1, 2.1, 0, 1)
+    ref = M.solve(g)
+    with M.Server(tuning=dict(workers=16), **SMALL) as small:
+        assert small.poll(small.submit(g), wait_ms=60_000).count == ref.count
+    first = M.Server(tuning=dict(workers=48), **SMALL)
+    second = M.Server(tuning=dict(workers=48), **SMALL)
+    got = []
+    try:
+        for name, srv in (("second", second), ("first", first)):
+            print(f"[gpu] request to the {name} server", flush=True)
+            r = srv.poll(srv.submit(g), wait_ms=20_000)
+            got.append((r.count, r.hash) if r else None)
+    finally:
+        # at the same time: a server's end waits for the other's kernel
+        ends = [threading.Thread(target=srv.close) for srv in (first, second)]
+        for t in ends:
+            t.start()
+        for t in ends:
+            t.join(60)
+    assert got == [(ref.count, ref.hash)] * 2
