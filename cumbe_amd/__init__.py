@@ -141,6 +141,8 @@ def lib() -> C.CDLL:
     L.mbe_server_get_stats.argtypes = [G, P(ServerStats)]
     L.mbe_server_destroy.argtypes = [G]
     L.mbe_server_destroy.restype = None
+    L.mbe_release_kept.argtypes = []
+    L.mbe_release_kept.restype = None
     for name in ("mbe_graph_load_bi", "mbe_graph_write_bi", "mbe_graph_from_edge_list",
                  "mbe_graph_from_csr", "mbe_graph_info", "mbe_graph_csr", "mbe_gen_chung_lu",
                  "mbe_gen_er_planted", "mbe_gen_batch_graph", "mbe_solve", "mbe_solve_list",
@@ -278,6 +280,11 @@ def solve(graph: Graph, variant: str = "cuMBE", tuning: Optional[dict] = None,
 def init() -> None:
     """mbe_init: set the engine up on device 0 (needed before solve_noalloc)."""
     _check(lib().mbe_init())
+
+
+def release_kept() -> None:
+    """mbe_release_kept: free the launch buffers that closed servers left."""
+    lib().mbe_release_kept()
 
 
 def solve_noalloc(dev_graph: int, info: PackedGraph, variant: str = "cuMBE",

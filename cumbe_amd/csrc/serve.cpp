@@ -34,8 +34,8 @@ using namespace mbe::host;
 // and that one ends when its owner says so. So a server takes the set only when
 // it holds all that its launches need (it allocates and frees nothing then), and
 // the set is freed, under the lock that counts the servers, only while none is
-// alive: by a server that cannot use it, and by an allocation of this library
-// that fails.
+// alive: by a server that cannot use it, by an allocation of this library that
+// fails, and by mbe_release_kept.
 constexpr size_t kKeepBytes = (size_t)16 << 30;
 struct Kept {
     std::mutex m;
@@ -607,5 +607,7 @@ void mbe_server_destroy(mbe_server* S) {
     free_server(S);
     delete S;
 }
+
+void mbe_release_kept(void) { (void)give_back_kept(); }
 
 }  // extern "C"

@@ -325,8 +325,14 @@ mbe_status mbe_server_submit(mbe_server* s, const mbe_graph* g, mbe_variant vari
 mbe_status mbe_server_poll(mbe_server* s, uint64_t ticket, int wait_ms, mbe_request_result* out);
 mbe_status mbe_server_get_stats(mbe_server* s, mbe_server_stats* out);
 /* Finish every admitted and queued request, close the kernel's mailbox,
- * wait for the kernel to drain, release the device buffers. */
+ * wait for the kernel to drain, release the device buffers. The launch buffers
+ * (9.4 GB at the default launch) are kept for the next server, one set of at
+ * most 16 GiB; another user of the device gets them after mbe_release_kept. */
 void mbe_server_destroy(mbe_server* s);
+/* Free the launch buffers that destroyed servers left. Does nothing while a
+ * server is alive. An allocation of the library that fails does this by
+ * itself. */
+void mbe_release_kept(void);
 
 #ifdef __cplusplus
 }

@@ -1,6 +1,7 @@
 """GPU tests of the launch buffers that pass from a destroyed server to the next
 one: servers that need more, less or the same as the one before, with a solve
 in between, all give the solve's result; and two servers at a time."""
+import ctypes
 import threading
 
 import pytest
@@ -56,3 +57,28 @@ def test_larger_server_beside_a_running_one():
         for t in ends:
             t.join(60)
     assert got == [(ref.count, ref.hash)] * 2
+
+
+def test_release_gives_the_buffers_back():
+    """What a destroyed server keeps goes back to the device on request, and
+    stays while a server is alive."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    g = M.Graph.chung_lu(300, 150, 1500, 2.1, 2.1, 0, 1)
+    ref = M.solve(g)
+    M.release_kept()
+    before = free_bytes()
+    with M.Server(tuning=dict(workers=256, arena_words=1 << 20), **SMALL) as srv:
+        assert srv.poll(srv.submit(g), wait_ms=60_000).count == ref.count
+    assert before - free_bytes() >= 256 * 8 << 20  # the arenas
+    with M.Server(tuning=dict(workers=256, arena_words=1 << 20), **SMALL) as srv:
+        M.release_kept()
+        assert srv.poll(srv.submit(g), wait_ms=60_000).count == ref.count
+        M.release_kept()
+    M.release_kept()
+    assert before - free_bytes() < 64 << 20
