@@ -830,21 +830,30 @@ mbe_status mbe_solve_noalloc(const void* dev_graph, const mbe_packed_graph* info
     uint32_t launches = 0, used_workers = 0;
     mbe::KParams kp{};
     for (int pass = 0; n_tasks > 0; pass++) {
-        const bool tree = pass == 0 && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
         if (pass >= mbe::kMaxPasses + (kp.twins ? 1 : 0))
             return fail(MBE_ERANGE, "root subproblem does not fit an arena of the scratch");
-        const uint64_t slot_words = ring_slot_words(arena_words);
-        const uint64_t w_slots = up4(kNoAllocSlots * slot_words);
+        const uint64_t room = fixed < mbe::kNoAllocWords ? mbe::kNoAllocWords - fixed : 0;
+        uint64_t per_worker = up4(arena_words) + up4(m.mark_words()) + up4((m.cpos_len() + 1) / 2);
         // the tree engine's hand-over: a slot and, of the control block, a
-        // flag line and a share of the idle map per worker
-        const uint64_t tslot_words = std::min(tree_slot_words(arena_words), kNoAllocTreeSlotWords);
-        const uint64_t per_worker = up4(arena_words) + up4(m.mark_words()) +
-                                    up4((m.cpos_len() + 1) / 2) + (tree ? tslot_words + 32 : 0);
-        const uint64_t fit = fixed + w_slots + 64 < mbe::kNoAllocWords
-                                 ? (mbe::kNoAllocWords - fixed - w_slots - 64) / per_worker : 0;
+        // flag line and a share of the idle map per worker. More workers than
+        // that leaves room for get smaller slots, or, when those would hold
+        // next to no level, the general engine and its ring
+        bool tree = pass == 0 && !(tu.flags & MBE_FLAG_REFERENCE_TREE);
+        uint64_t tslot_words = std::min(tree_slot_words(arena_words), kNoAllocTreeSlotWords);
+        if (tree && fixed_workers && room > 64) {
+            const uint64_t each = (room - 64) / workers;
+            const uint64_t left = each > per_worker + 32 ? (each - per_worker - 32) & ~(uint64_t)31 : 0;
+            tslot_words = std::min(tslot_words, left);
+            tree = tslot_words >= kMinTreeSlotWords;
+        }
+        const uint64_t slot_words = ring_slot_words(arena_words);
+        const uint64_t w_slots = tree ? 0 : up4(kNoAllocSlots * slot_words);
+        if (tree) per_worker += tslot_words + 32;
+        const uint64_t extra = w_slots + (tree ? 64 : 0);
+        const uint64_t fit = room > extra ? (room - extra) / per_worker : 0;
         if (fixed_workers && pass == 0 && workers > fit)
             return fail(MBE_ERANGE, std::to_string(workers) + " workers need " +
-                                        std::to_string((fixed + w_slots + workers * per_worker) * 8) +
+                                        std::to_string((fixed + extra + workers * per_worker) * 8) +
                                         " bytes of scratch; the allocation-free solve has " +
                                         std::to_string(mbe::kNoAllocBytes));
         const uint32_t nw = (uint32_t)std::min<uint64_t>(workers, fit);

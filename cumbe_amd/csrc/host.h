@@ -137,6 +137,7 @@ inline uint64_t tree_slot_words(uint64_t arena_words) {
     return std::min<uint64_t>(std::max<uint64_t>(1024, arena_words), kTreeSlotWords);
 }
 constexpr uint64_t kNoAllocTreeSlotWords = 4096;
+constexpr uint64_t kMinTreeSlotWords = 512;
 // allocation-free solve: deque slots and default arena (u64 words)
 constexpr uint32_t kNoAllocSlots = 64;
 constexpr uint64_t kNoAllocArenaWords = 1u << 15;

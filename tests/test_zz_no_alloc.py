@@ -105,3 +105,15 @@ def test_list_mode_root_at_the_default_arena():
     ref = O.solve(n_u, n_v, off, adj)
     assert (r.count, r.hash, r.launches) == (ref.count, ref.hash, 2)
     assert before - free_bytes() < 8 << 30
+
+
+@pytest.mark.parametrize("tuning", [{"workers": 850}, {"workers": 940},
+                                    {"workers": 40000, "arena_words": 512},
+                                    {"workers": 60000, "arena_words": 256}], ids=str)
+def test_many_workers_fit_the_scratch(tuning):
+    """Explicit worker counts that the arenas, marks and rank tables leave room
+    for: hand-over slots shrink, or the general engine's ring takes their place."""
+    M.init()
+    say(f"noalloc {tuning}")
+    r = check(M.Graph.chung_lu(400, 300, 2500, 2.1, 2.1, 0, 11), "cuMBE", tuning)
+    assert r.workers == tuning["workers"]
