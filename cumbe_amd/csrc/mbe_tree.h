@@ -724,6 +724,11 @@ __device__ __forceinline__ uint32_t gather_bits(const u64* M, uint32_t Wc, uint3
     }
     return n;
 }
+// Lane i's word of L: word w0 + i.
+__device__ __forceinline__ u64 word_of(const u64* L, uint32_t W, uint32_t w0) {
+    const Here lane;
+    return w0 + lane() < W ? L[w0 + lane()] : 0;
+}
 // Words of L (W of them) that are not zero, packed as a tile word map;
 // returns how many, or kTileW + 1 when a tile cannot hold them.
 __device__ __forceinline__ uint32_t word_map(const u64* L, uint32_t W, u64& wmap) {
@@ -798,6 +803,34 @@ __device__ __forceinline__ int place_level(const Wide& S, u64* F, uint32_t pn, u
     return kToTile;
 }
 
+// fn(i, row word) for the words w0 + i, i in m, of candidate block b, a
+// candidate per lane; four loads in flight. m holds the words that L has bits
+// in: below a hub root L' is a few bits, each in a word of its own, of a
+// universe of many words. Five roots of 4,000 L bits against 900 candidates
+// (63 words, a level's L' some 80 bits): 502 ms of kernel with every word read,
+// 346 so; universes of a few words the same.
+template <class F>
+__device__ __forceinline__ void each_row(const Wide& S, uint32_t w0, uint32_t b, u64 m, F&& fn) {
+    const Here lane;
+    const u64* rows = S.rows + (size_t)w0 * S.ncs + b * 64 + lane();
+    while (__popcll(m) >= 4) {
+        uint32_t i[4];
+        u64 r[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            i[t] = __builtin_ctzll(m);
+            m &= m - 1;
+            r[t] = rows[(size_t)i[t] * S.ncs];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) fn(i[t], r[t]);
+    }
+    for (; m; m &= m - 1) {
+        const uint32_t i = __builtin_ctzll(m);
+        fn(i, rows[(size_t)i * S.ncs]);
+    }
+}
+
 // Walk the wide levels from level k until a child fits the tile (kToTile,
 // src set; its level is k + 1), an event is due (kEvent) or the problem is
 // finished (kDone). resume: level k's x in progress has just been handled.
@@ -847,6 +880,7 @@ __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide
         u64* Qc = Xc + Wc;
         for (uint32_t w = lane(); w < W; w += 64) Lc[w] = S.rows[(size_t)w * S.ncs + x] & L[w];
         wsync();
+        const u64 p0 = word_of(L, W, 0), c0 = word_of(Lc, W, 0);
         if (SEC) sec.mark(kSecLPrime);
         wk.words += (u64)W * S.nc;
         bool nonmax = false;
@@ -856,10 +890,13 @@ __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide
             u64 tm = 0;
             if (qw) {
                 u64 miss = 0, touch = 0;
-                for (uint32_t w = 0; w < W; w++) {
-                    const u64 r = S.rows[(size_t)w * S.ncs + b * 64 + lane()], l = Lc[w];
-                    miss |= l & ~r;
-                    touch |= r & l;
+                for (uint32_t w0 = 0; w0 < W; w0 += 64) {
+                    const u64 c = w0 ? word_of(Lc, W, w0) : c0;
+                    each_row(S, w0, b, __ballot(c != 0), [&](uint32_t i, u64 r) {
+                        const u64 l = rdlane64(c, i);
+                        miss |= l & ~r;
+                        touch |= r & l;
+                    });
                 }
                 if (__ballot(miss == 0) & qw) {
                     nonmax = true;
@@ -878,11 +915,14 @@ __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide
             u64 pm = 0;
             if (live) {
                 u64 out = 0, miss = 0, touch = 0;
-                for (uint32_t w = 0; w < W; w++) {
-                    const u64 r = S.rows[(size_t)w * S.ncs + b * 64 + lane()], l = Lc[w];
-                    out |= r & L[w] & ~l;
-                    miss |= l & ~r;
-                    touch |= r & l;
+                for (uint32_t w0 = 0; w0 < W; w0 += 64) {
+                    const u64 p = w0 ? word_of(L, W, w0) : p0, c = w0 ? word_of(Lc, W, w0) : c0;
+                    each_row(S, w0, b, __ballot(p != 0), [&](uint32_t i, u64 r) {
+                        const u64 l = rdlane64(c, i);
+                        out |= r & rdlane64(p, i) & ~l;
+                        miss |= l & ~r;
+                        touch |= r & l;
+                    });
                 }
                 const u64 dead = __ballot(out == 0);
                 if (!nonmax) {

@@ -8,6 +8,7 @@ a few rows in the middle have a hole. All rows have about the same degree, so a 
 windows before it and its Q those after it, up to d / s of each.
 """
 import os
+import random
 import re
 import subprocess
 import time
@@ -32,6 +33,16 @@ def windows(n, d, s, holes):
     gone = {n // 2 + i: i * s + d // 2 - i for i in range(holes)}
     edges = [(i, i * s + j) for i in range(n) for j in range(d) if gone.get(i) != j]
     return csr_from_edges(n, (n - 1) * s + d, edges)
+
+
+# (rows, columns, columns per row): universes of 10, 66 and 130 words below
+# which L' is a few bits, each in a word of its own
+SCATTERED = [(18, 5000, 600), (9, 40000, 4200), (8, 60000, 8300)]
+
+
+def scattered(n, cols, d):
+    rng = random.Random(n)
+    return csr_from_edges(n, cols, [(i, j) for i in range(n) for j in rng.sample(range(cols), d)])
 
 
 def case_id(c):
@@ -64,6 +75,30 @@ def test_tiles_emulated(case, emu, tmp_path):
         count, h, nodes, donated, stolen = emu(*opts, "bi", path)
         assert (count, h) == (ref.count, ref.hash), opts
         assert donated == stolen and nodes >= count
+
+
+@pytest.mark.parametrize("case", SCATTERED, ids=case_id)
+def test_scattered_levels_emulated(case, emu, tmp_path):
+    g = scattered(*case)
+    ref = O.solve(*g)
+    path = str(tmp_path / "s.bi")
+    M.Graph.from_csr(*g).write_bi(path)
+    for opts in (("-w", 4), ("-w", 8, "-l", 420, "-i", 1)):
+        count, h, _, donated, stolen = emu(*opts, "-S", 0, "bi", path)
+        assert (count, h) == (ref.count, ref.hash), opts
+        assert donated == stolen
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", SCATTERED, ids=case_id)
+def test_scattered_levels_on_gpu(case):
+    g = scattered(*case)
+    ref = O.solve(*g)
+    gg = M.Graph.from_csr(*g)
+    for t in ({"side": 0}, {"side": 0, "workers": 24, "donate_interval": 1, "lds_words": 420}):
+        print(f"scattered {case} tuning {t}", flush=True)
+        r = M.solve(gg, "cuMBE", t)
+        assert (r.count, r.hash) == (ref.count, ref.hash), t
 
 
 @pytest.mark.gpu
@@ -138,9 +173,7 @@ def test_node_budget_counts_nodes(emu, tmp_path):
     """The node budget is in nodes of the tree as they are reported, on wide
     levels too (some 300 candidates a root here): a budget that covers them
     does not stop the solve, a quarter of it does."""
-    import random
-    rng = random.Random(1)
-    g = csr_from_edges(600, 800, [(i, j) for i in range(600) for j in rng.sample(range(800), 8)])
+    g = scattered(600, 800, 8)
     ref = O.solve(*g)
     path = str(tmp_path / "sparse.bi")
     M.Graph.from_csr(*g).write_bi(path)
