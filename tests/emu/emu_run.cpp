@@ -27,6 +27,9 @@
 //          -G seed of the garbage that fills uncleared device buffers
 //          -D us: a late atomic (wave_emu.h) lingers up to us after the next
 //             one, by a random sequence of seed -G
+//          -E words: materialise into that many device words; checks that the
+//             records' hashes add up to the reported one
+//          -C 1: section clocks (prints their sum)
 //          -g 1: the general engine for the first pass, too
 //          -A ms: raise the abort flag ms after a pass starts (a time limit)
 //          -n nodes: node budget (prints "aborted" when it is reached)
@@ -57,13 +60,14 @@ struct Opt {
     uint32_t large_edges = 1u << 18, table_cap = 64, gap_us = 0, stale_ms = 0;
     uint32_t workers = 8, lds_words = 3072, slots = 64, cutoff = 0, ratio = 2, interval = 64,
              twins = 1, rb = 0, re = 0, rs = 1;
-    uint64_t arena_words = 1u << 18, budget = 0;
-    bool general = false;
+    uint64_t arena_words = 1u << 18, budget = 0, emit = 0;
+    bool general = false, sections = false;
 };
 
 template <int V>
 static void wave_fn(void* p) { mbe_persistent<V>(*(KParams*)p); }
-static void tree_fn(void* p) { mbe_tree<false, false>(*(KParams*)p); }
+template <bool SEC, bool EMIT>
+static void tree_fn(void* p) { mbe_tree<SEC, EMIT>(*(KParams*)p); }
 
 // Words of the emulated LDS past the launch's dynamic LDS hold this pattern
 // while a wave runs; a write beyond the budget changes one and is reported.
@@ -79,7 +83,8 @@ static uint32_t g_abort_ms = 0;
 static void run_pass(KParams& kp, uint32_t workers) {
     void (*fn)(void*) = kp.variant == 1 ? wave_fn<1> : kp.variant == 2 ? wave_fn<2>
                       : kp.variant == 3 ? wave_fn<3> : wave_fn<0>;
-    if (kp.tree) fn = tree_fn;
+    if (kp.tree)
+        fn = kp.emit_pos ? tree_fn<true, true> : kp.sections ? tree_fn<true, false> : tree_fn<false, false>;
     std::atomic<bool> pass_done{false};
     std::thread mon;
     if (g_progress_s && kp.progress)
@@ -373,6 +378,8 @@ int main(int argc, char** argv) {
             case 'T': o.table_cap = (uint32_t)v; break;
             case 'u': o.gap_us = (uint32_t)v; break;
             case 'G': g_fill_seed = emu::g_linger_seed = (uint64_t)v; break;
+            case 'E': o.emit = (uint64_t)v; break;
+            case 'C': o.sections = v != 0; break;
             case 'g': o.general = v != 0; break;
             case 'A': g_abort_ms = (uint32_t)v; break;
             case 'n': o.budget = (uint64_t)v; break;
@@ -429,6 +436,8 @@ int main(int argc, char** argv) {
     uint32_t workers = o.workers;
     unsigned launches = 0;
     uint64_t last_arena = 0;  // of the last pass
+    std::vector<uint64_t> emit(o.emit);
+    unsigned long long* emit_pos = (unsigned long long*)shared(zalloc(16), 2);
     KParams kp{};
     while (!tasks.empty()) {
         if (launches > kMaxPasses) { fprintf(stderr, "root does not fit any arena\n"); return 4; }
@@ -475,6 +484,12 @@ int main(int argc, char** argv) {
         kp.donate_interval = o.interval;
         kp.dq = dq;
         kp.progress = progress;
+        if (o.sections) kp.sections = ctl + 2 + kStatCount;
+        if (o.emit) {
+            kp.emit_pos = emit_pos;
+            kp.emit = emit.data();
+            kp.emit_cap = o.emit;
+        }
         tree_setup(kp, workers, o.twins && !o.general && !launches);
         run_pass(kp, workers);
         free(kp.tctl);
@@ -499,6 +514,23 @@ int main(int argc, char** argv) {
            res[0], res[1], st[kStatNodes], st[kStatDonated], st[kStatStolen], st[kStatDropped],
            launches, abort_flag ? " aborted" : "");
     printf("arena %llu\n", (unsigned long long)last_arena);
+    if (o.sections) {
+        unsigned long long t = 0;
+        for (int j = 0; j < kSecCount; j++) t += ctl[2 + kStatCount + j];
+        printf("ticks %llu\n", t);
+    }
+    if (o.emit && emit_pos[0] <= o.emit) {
+        uint64_t n = 0, h = 0;
+        for (uint64_t at = 0; at < emit_pos[0]; n++) {
+            const uint64_t nl = emit[at] & 0xffffffffu, nr = emit[at] >> 32, sr = emit[at + 1];
+            uint64_t sl = 0;
+            for (uint64_t j = 0; j < nl; j++) sl += emit[at + 2 + j];
+            h += p.r_is_u ? biclique_hash(sr, sl, nr, nl) : biclique_hash(sl, sr, nl, nr);
+            at += 2 + nl;
+        }
+        printf("records %llu hash 0x%016llx\n", (unsigned long long)n, (unsigned long long)h);
+        if (n != res[0] || h != res[1]) return 6;
+    }
     if (o.budget) printf("charged %llu\n", st[kStatNodeBudget]);
     return st[kStatDropped] ? 5 : 0;
 }

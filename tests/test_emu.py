@@ -2,10 +2,12 @@
 under the wave64 emulator (tests/emu/, one fiber per lane, waves on OS
 threads) and checked against the oracle.
 
-These tests exercise the device code's logic without a GPU: root
-localisation with Q reduction, candidate selection, the reverse and forward
-checks, twin pruning, compaction into nested problems, donation through the
-deque and the LDS spill. The GPU tests check the same source on gfx950.
+These tests exercise the device code's logic without a GPU. The first pass of
+a run is the tree engine's unless the reference's tree is asked for (-t 0) or
+the general engine for all passes (-g 1). The general engine's candidate
+selection, reverse and forward checks, twin pruning, compaction into nested
+problems and ring are exercised under those two, and in overflow passes. The
+GPU tests check the same source on gfx950.
 """
 import json
 import os
@@ -192,3 +194,64 @@ def test_random_tunings():
                 "-G", rng.randint(1, 10**6)]
         r = emu(*opts, "cl", *ga)
         assert (r["count"], r["hash"]) == (ref.count, ref.hash), (case, opts, ga)
+
+
+# The first pass runs on the tree engine, which takes neither the cutoff, the
+# compaction ratio nor the split, and the variants other than noWS alike. What
+# follows runs on the general engine (-g 1), as the roots do that the tree
+# engine leaves.
+GENERAL = ("-g", 1)
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+@pytest.mark.parametrize("opts", [(), ("-r", 4294967295), ("-r", 8), ("-c", 8), ("-p", 1)],
+                         ids=lambda o: "".join(map(str, o)) or "default")
+def test_general_engine(variant, opts):
+    """Pruned tree of the general engine: every variant with re-localisation
+    on, off and late, row tests for small sets, and forced list mode."""
+    args = (400, 300, 2500, 2.1, 2.1, 0, 11)
+    ref = O.solve(*M.Graph.chung_lu(*args).csr())
+    r = emu(*GENERAL, "-v", variant, "-l", 600, *opts, "cl", *args)
+    assert (r["count"], r["hash"]) == (ref.count, ref.hash)
+
+
+@pytest.mark.parametrize("opts", [("-i", 8), ("-i", 8, "-p", 1), ("-i", 64, "-x", 16), ("-i", 8, "-s", 4)],
+                         ids=lambda o: "".join(map(str, o)))
+def test_general_engine_ring(opts):
+    """Levels move through the ring of the general engine: at every look, from
+    list-mode roots, with early splitting, and with four slots."""
+    args = (6500, 1900, 0.008, 60, 8, 40, 0.05, 3)
+    ref = O.solve_roots(*M.Graph.er_planted(*args).csr(), begin=0, end=12, threads=4)
+    r = emu(*GENERAL, "-w", 8, "-e", 12, "-l", 600, *opts, "er", *args)
+    assert (r["count"], r["hash"]) == (ref.count, ref.hash)
+    assert r["donated"] == r["stolen"] > 0
+
+
+@pytest.mark.parametrize("opts", [("-E", 1 << 20), ("-C", 1), ("-E", 1 << 20, "-l", 420, "-i", 1),
+                                  ("-C", 1, "-l", 420, "-i", 1), (*GENERAL, "-E", 1 << 20),
+                                  (*GENERAL, "-C", 1)], ids=lambda o: "".join(map(str, o)))
+def test_records_and_clocks(opts):
+    """The kernels that materialise (the records' hashes add up to the one
+    reported, which emu_run checks) and that keep section clocks."""
+    args = (400, 300, 2500, 2.1, 2.1, 0, 11)
+    ref = O.solve(*M.Graph.chung_lu(*args).csr())
+    out = subprocess.run([EMU, "-w", "4", *map(str, opts), "cl", *map(str, args)], capture_output=True,
+                         text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert f"count {ref.count} hash {ref.hash:#018x}" in out.stdout
+    assert f"records {ref.count}" in out.stdout or int(re.search(r"ticks (\d+)", out.stdout).group(1)) > 0
+
+
+def test_serving_hands_over():
+    """Served requests whose roots are deep, the next ones published while
+    idle workers watch for levels: every step looks for one to hand a level."""
+    specs = [(120, 14, 0.7, 0, 0, 0, 0, s) for s in range(1, 5)]
+    refs = [O.solve(*M.Graph.er_planted(*s).csr()) for s in specs]
+    out = subprocess.run([EMU, "-w", "8", "-i", "1", "-S", "1", "-u", "30000", "serve",
+                          *("e" + ",".join(map(str, s)) for s in specs)], capture_output=True,
+                         text=True, timeout=300)
+    assert out.returncode == 0, out.stderr + out.stdout
+    for i, r in enumerate(refs):
+        assert f"req {i} count {r.count} hash {r.hash:#018x} err 0 done 1" in out.stdout
+    m = re.search(r"donated (\d+) stolen (\d+)", out.stdout)
+    assert m.group(1) == m.group(2) != "0"
