@@ -6,7 +6,9 @@ work-stealing deque, the two list-versus-bitmap cutoffs -- sparse_ratio (a
 root whose bit matrices would take more than this many words per local
 adjacency entry is localised as sorted lists) and list_cutoff (|P|+|Q| at or
 below which a node tests candidate rows instead of AND/OR-ing L' columns) --
-and the re-localisation ratio. Workers are single waves, so the workgroup
+and the re-localisation ratio. The last two act in the general engine alone,
+on roots that the tree engine leaves to a later pass, so the workloads here are
+searched without them (TREE_AXES). Workers are single waves, so the workgroup
 size is not a search axis. Coordinate descent from a start point: each trial is
 the mean of two runs and a move needs a 5 % gain (single runs of one
 configuration vary by several percent). Every trial runs under the engine's
@@ -26,7 +28,7 @@ import json
 import os
 import sys
 import time
-from typing import Callable, Dict, List, Optional
+from typing import Callable, List, Optional, Sequence
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CACHE = os.path.join(HERE, "tuning_cache.json")
@@ -43,6 +45,7 @@ GRID = {
     "compact_ratio": [2, 4, 0xFFFFFFFF],
     "sparse_ratio": [8, 32, 0xFFFFFFFF],
 }
+TREE_AXES = ("occupancy", "donate_interval", "sparse_ratio")
 START = {"occupancy": (2560, 8), "donate_interval": 32, "list_cutoff": 0, "compact_ratio": 2,
          "sparse_ratio": 0xFFFFFFFF}
 
@@ -74,8 +77,9 @@ def _store(key: str, tuning: dict, ms: float, trials: List[dict]) -> None:
 
 
 def tune(key: str, run: Callable[[dict], Optional[float]], budget_s: float,
-         start: Optional[dict] = None, repeats: int = 2, gain: float = 0.05) -> dict:
-    """Coordinate descent over GRID: run(tuning) returns kernel ms (None if it
+         start: Optional[dict] = None, repeats: int = 2, gain: float = 0.05,
+         axes: Optional[Sequence[str]] = None) -> dict:
+    """Coordinate descent over GRID (its axes named, or all): run(tuning) returns kernel ms (None if it
     failed), averaged over `repeats` runs; a neighbour replaces the current
     point when it is faster by more than `gain`. The cached and returned
     tuning is in engine terms (expand)."""
@@ -92,8 +96,8 @@ def tune(key: str, run: Callable[[dict], Optional[float]], budget_s: float,
     improved = True
     while improved and time.time() - t0 < budget_s:
         improved = False
-        for name, values in GRID.items():
-            for v in values:
+        for name in axes or GRID:
+            for v in GRID[name]:
                 if v == best[name] or time.time() - t0 > budget_s:
                     continue
                 cand = dict(best, **{name: v})
@@ -157,7 +161,7 @@ def main() -> None:
             with open(CACHE) as f, open(args.cache, "w") as g:
                 g.write(f.read())
         CACHE = args.cache
-    best = tune(args.workload, _workload(args.workload), args.budget_s)
+    best = tune(args.workload, _workload(args.workload), args.budget_s, axes=TREE_AXES)
     print(json.dumps({"workload": args.workload, "tuning": best}))
 
 

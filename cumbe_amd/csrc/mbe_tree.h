@@ -871,7 +871,9 @@ __device__ __forceinline__ int wide_walk(const KParams& kp, Walk& wk, const Wide
             resume = true;
             continue;
         }
-        // L', and a step costs about as much as four tile steps per word of P
+        // L'. A wide step counts for one tile step and for half a one per word of
+        // candidates; it takes longer than as many, so events are further apart
+        // in time here
         wk.steps += 1 + Wc / 2;
         u64* Fc = S.frame(k + 1);
         u64* Lc = Fc + kFrameHdr;

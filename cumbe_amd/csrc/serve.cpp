@@ -466,8 +466,10 @@ mbe_status make_server(mbe_server* S) {
                                   : 160 * 1024;
     // serving defaults: 8 MiB arenas per worker, so that every root of the
     // batched size distribution fits the kernel, and four 32 KiB workers per
-    // CU (the large requests' local problems stay in LDS; six 24 KiB workers
-    // raised their isolated latency by about 40 %)
+    // CU, with which 48 requests of that distribution take 1.1 ms each one at
+    // a time (mean) and 13 ms as a burst, and one of 1.5 M edges 45 ms alone;
+    // with six 24 KiB workers 1.6, 19 and 49, with eight 20 KiB workers 2.2, 28
+    // and 57, although those are faster on a batch
     if (!S->cfg.tuning.arena_words) S->cfg.tuning.arena_words = 1u << 20;
     if (!S->cfg.tuning.lds_words) S->cfg.tuning.lds_words = 4096;
     if (!S->cfg.tuning.waves_per_cu && !S->cfg.tuning.workers) S->cfg.tuning.waves_per_cu = 4;

@@ -42,7 +42,12 @@ typedef enum {
     MBE_EINTERNAL = -10    /* the engine's results failed a self-check */
 } mbe_status;
 
-/* The four algorithm variants of the reference (src/main.cu:121-122). */
+/* The four algorithm variants of the reference (src/main.cu:121-122). They
+ * give the same results. By default one pruned search runs for all of them,
+ * without hand-over of subtrees for MBE_NOWS; what else is said here holds under
+ * MBE_FLAG_REFERENCE_TREE and in the passes over the roots that the pruned
+ * search leaves (list mode suits them, or they exceed an arena), which run on
+ * the general engine. */
 typedef enum {
     MBE_CUMBE = 0, /* reverse scans + early-stop selection + work stealing */
     MBE_NORS = 1,  /* forward scans over N(v) for the Q check and expansion */
@@ -59,14 +64,15 @@ typedef struct {
     uint32_t waves_per_cu;   /* occupancy target used when workers == 0 */
     uint32_t lds_words;      /* per-worker LDS stack budget in u64 words */
     uint32_t arena_words;    /* per-worker HBM arena in u64 words */
-    uint32_t list_cutoff;    /* P/Q size at or below which nodes use row
-                                (sorted-list style) scans instead of
-                                column bitmaps; 0 = default */
+    uint32_t list_cutoff;    /* general engine: P/Q size at or below which
+                                nodes use row (sorted-list style) scans
+                                instead of column bitmaps; 0 = default */
     uint32_t donate_depth;   /* deepest level a worker donates from; 0 = any */
-    uint32_t compact_ratio;  /* re-localise a child subproblem when its universe
-                                shrank by this factor; 0 = default (2),
-                                UINT32_MAX = never */
-    uint32_t donate_interval;/* nodes between a worker's donation checks; 0 = 32 */
+    uint32_t compact_ratio;  /* general engine: re-localise a child subproblem
+                                when its universe shrank by this factor;
+                                0 = default (2), UINT32_MAX = never */
+    uint32_t donate_interval;/* vertices tested between a worker's donation
+                                checks; 0 = 32 */
     int32_t side;            /* -1 reference side choice, 0 enumerate U, 1 V */
     uint32_t flags;          /* MBE_FLAG_* */
     /* Root subset: ranks r with root_begin <= r < root_end (0 = all) and
@@ -74,9 +80,10 @@ typedef struct {
      * stride shards one graph across devices or processes: the partial
      * counts and hashes of the shards add up to the whole. Single graph only. */
     uint32_t root_begin, root_end, root_stride;
-    /* Watchdog: stop after about max_nodes tree nodes or time_limit_ms of
-     * wall time (0 = none); the solve then returns MBE_ETIMEOUT and the
-     * result holds the partial count, hash and node total. */
+    /* Watchdog: stop after about max_nodes tree nodes (as mbe_result.nodes
+     * counts them) or time_limit_ms of wall time (0 = none); the solve then
+     * returns MBE_ETIMEOUT and the result holds the partial count, hash and
+     * node total. */
     uint64_t max_nodes;
     double time_limit_ms;
     /* List-versus-bitmap cutoff of root localisation: a root with at most 8
@@ -85,10 +92,11 @@ typedef struct {
      * adjacency lists instead (the reference's list scans,
      * src/mbe_cuMBE.cuh:188-236,345-390): bit rows only for its P
      * candidates, the candidates of each L vertex and the L vertices of each
-     * candidate as lists. Such a root's tree (at most 256 nodes) is searched
-     * by one worker. 0 = default (8), UINT32_MAX = never. */
+     * candidate as lists, in a pass of its own on the general engine. Such a
+     * root's tree (at most 256 nodes) is searched by one worker. 0 = default
+     * (8), UINT32_MAX = never. */
     uint32_t sparse_ratio;
-    /* A task (root or stolen subtree) that has run this many tree nodes
+    /* General engine: a task (root or stolen subtree) that has run this many tree nodes
      * hands part of its work to the deque at its donation checks while fewer
      * than 64 tasks wait there, even when no worker is idle, so that heavy
      * roots spread before the tail. 0 = default (4096), UINT32_MAX = only
@@ -104,8 +112,10 @@ typedef struct {
                               file ids' terms (cumbe_amd/csrc/hash.h) */
     double kernel_ms;      /* HIP-event time of the enumeration kernels */
     double total_ms;       /* host wall time incl. preprocessing and copies */
-    uint64_t nodes;        /* enumeration-tree nodes visited */
-    uint64_t donated;      /* subtree tasks donated through the deque */
+    uint64_t nodes;        /* enumeration-tree nodes; of the pruned tree one per
+                              biclique and one per root that gives none, with
+                              MBE_FLAG_REFERENCE_TREE all that are visited */
+    uint64_t donated;      /* subtree tasks handed to another worker */
     uint32_t launches;     /* kernel launches used */
     uint32_t workers;      /* workers used */
     /* Time per kernel section summed over workers, in 10 ns ticks, filled
@@ -129,10 +139,11 @@ typedef struct {
  * reference's DEVARIANCE build (src/mbe_noES.cuh:49-55); read it with
  * mbe_last_worker_busy. Implies MBE_FLAG_SECTIONS. */
 #define MBE_FLAG_VARIANCE 2u
-/* Walk exactly the reference's search tree. By default a candidate whose
- * neighbourhood within the current L equals that of the vertex just
- * selected is dropped from P (iMBEA's rule, which the reference leaves
- * out): each such candidate would only yield a non-maximal leaf. The
+/* Walk exactly the reference's search tree, in the given variant. By default
+ * a candidate whose neighbourhood within the current L lies inside that of a
+ * vertex already handled is dropped from P (where they are equal, this is
+ * iMBEA's rule, which the reference leaves out): each such candidate would
+ * only yield non-maximal nodes. The
  * bicliques reported are the same either way; the tree and the time are
  * not. In the serving loop, set it in mbe_server_config.tuning.flags. */
 #define MBE_FLAG_REFERENCE_TREE 4u
@@ -224,14 +235,14 @@ mbe_status mbe_graph_pack(const mbe_graph* g, int side, void* out, uint64_t cap_
  *
  * dev_graph is device memory holding what mbe_graph_pack wrote (described
  * by *info); the caller owns it and the result. Every other buffer the
- * kernels use -- control words, the deque and its slots, task lists, the
+ * kernels use -- control words, hand-over slots, task lists, the
  * per-worker arenas, marks and rank tables -- is carved out of one static
  * device array of MBE_NOALLOC_SCRATCH_BYTES, so the call makes no hipMalloc,
  * hipFree or other allocating call. mbe_init must have run (MBE_EINVAL
  * otherwise). Defaults: 32 K-word (256 KiB) arenas and as many workers as
  * fit, up to mbe_solve's count; roots whose local problem exceeds an arena
- * run in follow-up passes with 16 times larger arenas and fewer workers
- * inside the same array. A tuning or graph whose buffers do not fit the
+ * run in follow-up passes, at the same size first and then with 16 times
+ * larger arenas and fewer workers, inside the same array. A tuning or graph whose buffers do not fit the
  * array returns MBE_ERANGE; MBE_FLAG_VARIANCE returns MBE_EINVAL. The array
  * is shared by every call on a device and keeps the last call's contents
  * (each call clears what must start at zero); calls are serialised by the
@@ -248,7 +259,7 @@ mbe_status mbe_batch_solve(const mbe_graph* const* graphs, size_t n, mbe_variant
                            mbe_result* total);
 
 /* Batch plan: the graphs are prepared and uploaded once into a device arena
- * owned by the plan, and the first pass (control clears, deque reset, the
+ * owned by the plan, and the first pass (control clears and the
  * persistent launch over every root of every graph) is captured into a HIP
  * graph that each run replays. Roots whose local problem exceeds a worker's
  * arena are finished by eager follow-up launches, as in mbe_batch_solve.
@@ -272,8 +283,8 @@ void mbe_batch_plan_free(mbe_batch_plan* plan);
  * into pinned staging memory, reserves its place in the device data ring and
  * publishes a mailbox record. An idle wave of the running kernel copies the
  * CSR in and appends the request's roots to the shared task space, so a
- * request starts while earlier ones are still running and its subtrees share
- * the work-stealing deque with theirs. A request completes when its own last
+ * request starts while earlier ones are still running and its subtrees go to
+ * the same idle workers as theirs. A request completes when its own last
  * task does: the kernel raises its host-mapped completion flag. Requests for
  * another variant than cuMBE, or whose local problems exceed the serving
  * workers' arenas, run through mbe_solve in their turn, between two kernel
