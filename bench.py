@@ -148,7 +148,7 @@ def serving_leg(duration, rates):
 
 def traffic_from_profiles():
     """HBM bytes per launch measured by rocprofv3 --pmc (committed summary)."""
-    path = os.path.join(ROOT, "profiles", "mbe_persistent_c1_roots400.pmc.txt")
+    path = os.path.join(ROOT, "profiles", "mbe_tree_c1_roots400.pmc.txt")
     if not os.path.exists(path):
         return None
     m = re.search(r"^\s*hbm_bytes_per_launch:\s*([0-9.eE+]+)", open(path).read(), re.M)
@@ -339,8 +339,9 @@ def main():
             "traffic": traffic,
             "traffic_GBps": traffic / launch_s / 1e9 if traffic else None,
             "algorithmic_bytes_per_launch": op_bytes,
-            "limiter": ("issue and latency of one wave's chain of vertex tests (two waves per "
-                        "SIMD, register-limited); the operand words are served from registers"),
+            "limiter": ("one wave's chain of vertex tests, two waves per SIMD (register-limited): "
+                        "waves issue 39 % of their cycles and wait 53 %, VALUs are busy 39 %; "
+                        "the operand words are served from registers"),
             "launch_ms": launch_ms,
             "reference_equivalent_GBps": ref_gbps,
             "reference_work_entries": w_alg,
