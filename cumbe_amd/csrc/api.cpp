@@ -999,6 +999,8 @@ mbe_status capture_pass0(Engine& E, mbe_batch_plan* p) {
     return MBE_OK;
 }
 
+// Whether the capture is still what a run needs: its buffers, and progress
+// reports when they are asked for.
 bool capture_current(const mbe_batch_plan* p) {
     const mbe::KParams& kp = p->pass0.kp;
     return p->pass0.exec && kp.arena == p->b.arena.as<uint64_t>() &&
@@ -1008,7 +1010,8 @@ bool capture_current(const mbe_batch_plan* p) {
            kp.slots == p->b.slots.as<uint64_t>() &&
            kp.dq == p->b.dq.as<unsigned long long>() &&
            kp.tctl == p->b.tctl.as<unsigned long long>() &&
-           kp.tslots == p->b.tslots.as<uint64_t>();
+           kp.tslots == p->b.tslots.as<uint64_t>() &&
+           (kp.progress != nullptr) == (getenv("MBE_PROGRESS") != nullptr);
 }
 
 }  // namespace

@@ -160,3 +160,22 @@ def test_graphs_the_oracle_did_not_finish():
             say(f"seed {r['seed']} {v}")
             x = M.solve(g, v)
             assert (x.count, f"{x.hash:#018x}") == (r["count"], r["hash"]), (r["seed"], v)
+
+
+def test_plan_reports_progress_when_asked_later(monkeypatch, capfd):
+    """MBE_PROGRESS set after a plan was made: its runs report what the workers
+    have done, and no longer once it is unset."""
+    rows = [r for r in c3_rows() if r[1] is not None and 5_000_000 <= r[3] <= 10 ** 11][:256]
+    plan = M.BatchPlan([M.Graph.batch_graph(r[0]) for r in rows], "cuMBE")
+    plan.run()
+    monkeypatch.setenv("MBE_PROGRESS", "0.001")
+    per, _ = plan.run()
+    lines = [x for x in capfd.readouterr().err.splitlines() if x.startswith("[mbe] pass 0")]
+    say("\n".join(lines[-2:]))
+    assert lines and int(lines[-1].split(", ")[1].split("/")[0]) > 0
+    monkeypatch.delenv("MBE_PROGRESS")
+    again, _ = plan.run()
+    assert not [x for x in capfd.readouterr().err.splitlines() if x.startswith("[mbe]")]
+    assert [(r.count, r.hash) for r in per] == [(r[1], r[2]) for r in rows] == \
+        [(r.count, r.hash) for r in again]
+    plan.close()
